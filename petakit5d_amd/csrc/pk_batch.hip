@@ -53,6 +53,12 @@ struct Group {
 template <class T>
 using Pass = std::map<std::array<int64_t, 6>, Group<T>>;
 
+// A row pass: chunks of the three-pass form and of the two-pass form.
+struct RowPass {
+    Pass<XChunk> rows;
+    Pass<FoldX> fold;
+};
+
 int64_t smooth_up(int64_t n) {
     while (!smooth235(n)) ++n;
     return n;
@@ -169,7 +175,7 @@ size_t pk_ctx_impl::chunk_prepare(Chunk& c, const pk_vol& in, const pk_vol& out,
     c.out_bytes = (c.o.save16bit ? 2 : 4) * (size_t)(c.d[0] * c.d[1] * c.d[2]);
     const VolPlan& vp = *c.vp;
     const size_t esz = c.u16 ? 2 : 4;
-    const int64_t nxb = (vp.n2 * vp.n3 + vp.x.tile - 1) / vp.x.tile;
+    const int64_t nxb = vp.x_blocks();
     size_t need = 2 * align_up(sizeof(float) * vp.N) + align_up(sizeof(float2) * vp.S);
     if (c.method == 0) need += 3 * align_up(sizeof(float) * vp.N) + align_up(sizeof(double) * 2 * nxb) + kAlign;
     if (c.in_host) need += align_up(esz * (size_t)(c.d[0] * c.d[1] * c.d[2]));  // staging, caller's layout
@@ -192,7 +198,7 @@ void pk_ctx_impl::chunk_place(Chunk& c, char* base, hipStream_t copy_stream) {
     c.J = reinterpret_cast<float*>(take(sizeof(float) * vp.N));
     c.A = reinterpret_cast<float2*>(take(sizeof(float2) * vp.S));
     if (c.method == 0) {
-        const int64_t nxb = (vp.n2 * vp.n3 + vp.x.tile - 1) / vp.x.tile;
+        const int64_t nxb = vp.x_blocks();
         c.J3 = reinterpret_cast<float*>(take(sizeof(float) * vp.N));
         c.Y = reinterpret_cast<float*>(take(sizeof(float) * vp.N));
         c.J4 = reinterpret_cast<float*>(take(sizeof(float) * vp.N));
@@ -268,8 +274,28 @@ void pk_ctx_impl::run_step(std::vector<Chunk*>& act) {
         a.spec = c.A;
         return a;
     };
-    auto add_x = [&](Pass<XChunk>& ps, const Chunk& c, const XArgs& a) {
+    // chunks of the two-pass form: grouped by mode and block shape
+    auto add_fold = [&](auto& ps, const std::array<int64_t, 6>& key, const auto& f, unsigned nt, size_t lds,
+                        int64_t blocks) {
+        auto& g = ps[key];
+        g.mode = (int)key[1];
+        g.chunks.push_back(f);
+        g.starts.push_back(g.starts.back() + blocks);
+        g.block = nt;
+        g.lds = lds;
+    };
+    auto add_x = [&](RowPass& rp, const Chunk& c, const XArgs& a) {
         const VolPlan& vp = *c.vp;
+        if (vp.fold.on) {
+            const FoldPlan& fp = vp.fold;
+            FoldX f = fp.x;
+            f.a = a;
+            f.tw = vp.x.fp.tw;
+            f.twy = vp.y.fp.tw;
+            add_fold(rp.fold, {(int64_t)fp.xnt, a.mode, (int64_t)fp.xlds, 0, 0, 0}, f, fp.xnt, fp.xlds, fp.xblocks);
+            return;
+        }
+        Pass<XChunk>& ps = rp.rows;
         // chunks whose rows have a compile-time kernel are grouped by row length
         const int ctk = vp.packed ? vp.x.fp.L : -vp.x.fp.L;  // compile-time kernel key (odd rows negative)
         const int ctL = (vp.x.block.x == 256 && xrow_available(ctk, vp.x.fp.E)) ? ctk : 0;
@@ -291,11 +317,22 @@ void pk_ctx_impl::run_step(std::vector<Chunk*>& act) {
         const VolPlan& vp = *c.vp;
         const int ctk = vp.packed ? vp.x.fp.L : -vp.x.fp.L;
         const bool ok = c.u16 && c.numit >= (c.method == 1 ? 2 : 1) && !(c.o.damp_factor > 1) &&
-                        vp.x.block.x == 256 && xrow_available(ctk, vp.x.fp.E);
+                        (vp.fold.on || (vp.x.block.x == 256 && xrow_available(ctk, vp.x.fp.E)));
         return ok ? reinterpret_cast<uint16_t*>(c.I) : nullptr;
+    };
+    auto add_conv = [&](Pass<FoldC>& ps, const Chunk& c, int mode, const float2* otf) {
+        const VolPlan& vp = *c.vp;
+        const FoldPlan& fp = vp.fold;
+        FoldC f = fp.c;
+        f.data = c.A;
+        f.otf = otf;
+        f.twy = vp.y.fp.tw;
+        f.twz = vp.z.fp.tw;
+        add_fold(ps, {(int64_t)fp.cnt, mode, (int64_t)fp.clds, 0, 0, 0}, f, fp.cnt, fp.clds, fp.cblocks);
     };
     auto add_col = [&](Pass<ColChunk>& ps, const Chunk& c, int axis, int mode, const float2* otf) {
         const VolPlan& vp = *c.vp;
+        if (vp.fold.on) return;  // its two passes hold every strided step
         const AxisLaunch& ax = axis == 2 ? vp.y : vp.z;
         if (ax.fp.L == 1 && (mode == CM_FWD || mode == CM_INV)) return;
         ColArgs a{};
@@ -362,7 +399,8 @@ void pk_ctx_impl::run_step(std::vector<Chunk*>& act) {
             load[best] += act[i]->vp->N;
         }
     }
-    Pass<XChunk> prep[kSets], biggs_y[kSets], ratio[kSets], update[kSets];
+    RowPass prep[kSets], biggs_y[kSets], ratio[kSets], update[kSets];
+    Pass<FoldC> fc1[kSets], fc2[kSets];
     Pass<ColChunk> yf[kSets], zc1[kSets], yi[kSets], zc2[kSets];
     std::vector<LamChunk> lam;
     for (size_t ci = 0; ci < act.size(); ++ci) {
@@ -396,7 +434,7 @@ void pk_ctx_impl::run_step(std::vector<Chunk*>& act) {
         const int kn = c.k + 1;        // the iteration this step runs
         if (c.method == 0) {
             if (kn > 2)
-                lam.push_back(LamChunk{c.part, (int)((c.vp->n2 * c.vp->n3 + c.vp->x.tile - 1) / c.vp->x.tile), c.lam});
+                lam.push_back(LamChunk{c.part, (int)c.vp->x_blocks(), c.lam});
             XArgs a = base_x(c, XM_BIGGS_Y);
             a.J = c.par ? c.J3 : c.J;
             a.J3 = c.par ? c.J : c.J3;
@@ -405,6 +443,10 @@ void pk_ctx_impl::run_step(std::vector<Chunk*>& act) {
             add_x(biggs_y[si], c, a);
         }
         const int cax = c.vp->conv_axis, oax = cax == 3 ? 2 : 3;  // pass order of the chunk's plan
+        if (c.vp->fold.on) {
+            add_conv(fc1[si], c, CM_CONV, c.Hf);
+            add_conv(fc2[si], c, c.method == 1 ? CM_CONV : CM_CONVJ, c.method == 1 ? c.Hb : c.Hf);
+        }
         add_col(yf[si], c, oax, CM_FWD, nullptr);
         add_col(zc1[si], c, cax, CM_CONV, c.Hf);
         add_col(yi[si], c, oax, CM_INV, nullptr);
@@ -438,10 +480,12 @@ void pk_ctx_impl::run_step(std::vector<Chunk*>& act) {
         }
     }
     for (int k = 0; k < nset; ++k) {
-        seal(prep[k]);
-        seal(biggs_y[k]);
-        seal(ratio[k]);
-        seal(update[k]);
+        for (RowPass* rp : {&prep[k], &biggs_y[k], &ratio[k], &update[k]}) {
+            seal(rp->rows);
+            seal(rp->fold);
+        }
+        seal(fc1[k]);
+        seal(fc2[k]);
         seal(yf[k]);
         seal(zc1[k]);
         seal(yi[k]);
@@ -473,8 +517,16 @@ void pk_ctx_impl::run_step(std::vector<Chunk*>& act) {
     PK_HIP(hipEventRecord(ws.tab_ev[slot], stream));
     char* tab = ws.tab_dev[slot].as<char>();
 
-    auto run_x = [&](const Pass<XChunk>& ps, const char* name, hipStream_t st) {
-        for (auto& kv : ps) {
+    auto run_x = [&](const RowPass& rp, const char* name, hipStream_t st) {
+        for (auto& kv : rp.fold) {
+            const auto& g = kv.second;
+            hipEvent_t e0 = prof_mark();
+            PK_HIP(launch_foldx(g.block, dim3((unsigned)g.starts.back()), g.lds, st, g.chunks[0], g.mode,
+                                reinterpret_cast<const FoldX*>(tab + g.dev_off),
+                                reinterpret_cast<const int64_t*>(tab + g.start_off), (int)g.chunks.size()));
+            prof_done(name, 0, e0);
+        }
+        for (auto& kv : rp.rows) {
             const auto& g = kv.second;
             hipEvent_t e0 = prof_mark();
             const XChunk* chd = reinterpret_cast<const XChunk*>(tab + g.dev_off);
@@ -498,6 +550,16 @@ void pk_ctx_impl::run_step(std::vector<Chunk*>& act) {
             prof_done(name, 0, e0);
         }
     };
+    auto run_f = [&](const Pass<FoldC>& ps, const char* name, hipStream_t st) {
+        for (auto& kv : ps) {
+            const auto& g = kv.second;
+            hipEvent_t e0 = prof_mark();
+            PK_HIP(launch_foldc(g.block, dim3((unsigned)g.starts.back()), g.lds, st, g.chunks[0], g.mode,
+                                reinterpret_cast<const FoldC*>(tab + g.dev_off),
+                                reinterpret_cast<const int64_t*>(tab + g.start_off), (int)g.chunks.size()));
+            prof_done(name, 0, e0);
+        }
+    };
     if (!lam.empty()) {
         hipLaunchKernelGGL(k_lambda_batch, dim3((unsigned)lam.size()), dim3(256), 0, stream,
                            reinterpret_cast<const LamChunk*>(tab + lam_off), kEpsF);
@@ -516,10 +578,12 @@ void pk_ctx_impl::run_step(std::vector<Chunk*>& act) {
         hipStream_t st = k == 0 ? stream : side[k - 1];
         run_x(prep[k], "b_x_prep", st);
         run_x(biggs_y[k], "b_x_biggs_y", st);
+        run_f(fc1[k], "b_yz_conv", st);
         run_c(yf[k], "b_y_fwd", st);
         run_c(zc1[k], "b_z_conv", st);
         run_c(yi[k], "b_y_inv", st);
         run_x(ratio[k], "b_x_ratio", st);
+        run_f(fc2[k], "b_yz_conv", st);
         run_c(yf[k], "b_y_fwd", st);
         run_c(zc2[k], "b_z_conv", st);
         run_c(yi[k], "b_y_inv", st);

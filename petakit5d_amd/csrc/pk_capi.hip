@@ -214,7 +214,7 @@ pk_status pk_psf2otf(pk_ctx* c, const float* psf, const int64_t pd[3], const int
         const pk::VolPlan& vp = c->plan(od[0], od[1], od[2]);
         pk::DevBuf spec;
         c->alloc(spec, sizeof(float2) * (size_t)vp.S);
-        c->build_otf(vp, psf, pd, spec.as<float2>());
+        c->build_otf(vp.three_pass(), psf, pd, spec.as<float2>());  // natural frequency order
         std::vector<float2> h((size_t)vp.S);
         PK_HIP(hipMemcpy(h.data(), spec.p, sizeof(float2) * (size_t)vp.S, hipMemcpyDeviceToHost));
         // expand the half spectrum with Hermitian symmetry into MATLAB's full OTF

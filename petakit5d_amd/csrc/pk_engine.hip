@@ -194,6 +194,8 @@ struct Tune {
     // PK_TUNE_COL_CANDS: strided-axis shapes the autotuner times per axis, best-ranked first
     // (64 chunks, OMW-2 Gvoxel/s: 4 -> 17.5, 8 -> 17.0)
     int col_cands = 4;
+    // a pinned launch shape names the three-pass kernels: the two-pass form is off
+    bool pinned() const { return generic_x || e[0] || e[1] || e[2] || t[1] || t[2]; }
     Tune() {
         if (const char* v = std::getenv("PK_CHUNK_STREAMS")) streams = std::max(1, std::min(8, std::atoi(v)));
         if (const char* v = std::getenv("PK_TUNE_COL_CANDS")) col_cands = std::max(1, std::min(16, std::atoi(v)));
@@ -471,7 +473,7 @@ static bool col_axis(int L, int E, int nt, int T, AxisLaunch& ax) {
 
 // Tuned shapes per padded size, shared by the process's contexts and kept in
 // the text file PK_TUNE_FILE when set (one line per size:
-// n1 n2 n3  xE  yE yNT yT  zE zNT zT  conv_axis).
+// n1 n2 n3  xE  yE yNT yT  zE zNT zT  conv_axis; xE < 0: see apply_shapes).
 struct Wisdom {
     std::mutex mu;
     std::map<std::vector<int64_t>, std::array<int, 8>> table;
@@ -507,8 +509,13 @@ struct Wisdom {
 };
 
 // Launch shapes of one wisdom line {xE, yE, yNT, yT, zE, zNT, zT, conv_axis}
-// applied to a plan; false (plan unchanged) when a shape is infeasible.
-bool pk_ctx_impl::apply_shapes(VolPlan& vp, const std::array<int, 8>& v) {
+// applied to a plan; false (plan unchanged) when a shape is infeasible.  They
+// are the three-pass form's; xE < 0: and the size runs that form (measured
+// faster, or pinned), instead of the two-pass form where there is one.
+bool pk_ctx_impl::apply_shapes(VolPlan& vp, const std::array<int, 8>& line) {
+    std::array<int, 8> v = line;
+    const bool three = v[0] < 0;
+    v[0] = std::abs(v[0]);
     const int Lx = (int)(vp.packed ? vp.n1 / 2 : vp.n1);
     const bool ctx =
         !tune().generic_x && v[0] > 0 && Lx % v[0] == 0 && xrow_available(vp.packed ? Lx : -Lx, v[0]);
@@ -526,6 +533,7 @@ bool pk_ctx_impl::apply_shapes(VolPlan& vp, const std::array<int, 8>& v) {
     vp.z = az;
     vp.z.fp.tw = tz;
     vp.conv_axis = v[7];
+    if (three) vp.fold = FoldPlan{};
     vp.tuned = true;
     return true;
 }
@@ -533,13 +541,15 @@ bool pk_ctx_impl::apply_shapes(VolPlan& vp, const std::array<int, 8>& v) {
 void pk_ctx_impl::set_shapes(int64_t n1, int64_t n2, int64_t n3, const std::array<int, 8>& v) {
     const std::vector<int64_t> key{n1, n2, n3};
     VolPlan vp = plan(n1, n2, n3);
-    if (!apply_shapes(vp, v)) fail(PK_ERR_INVALID_ARG, "launch shapes not feasible for this size");
+    std::array<int, 8> pin = v;
+    pin[0] = -v[0];
+    if (v[0] < 1 || !apply_shapes(vp, pin)) fail(PK_ERR_INVALID_ARG, "launch shapes not feasible for this size");
     plans[key] = vp;
     clear_graphs();  // captured loops hold the old launch shapes
     Wisdom& w = Wisdom::get();
     std::lock_guard<std::mutex> lk(w.mu);
     w.load();
-    w.table[key] = v;
+    w.table[key] = pin;
 }
 
 // W_{n1}^k for k in [0, n1/2] (the split step of packed real rows), exact at
@@ -576,6 +586,7 @@ VolPlan pk_ctx_impl::plan_shapes(int64_t n1, int64_t n2, int64_t n3) const {
     vp.x = x_candidates(vp.row_len(), vp.packed)[0];
     vp.y = col_candidates((int)n2, 1)[0];
     vp.z = col_candidates((int)n3, 2)[0];
+    if (!tune().pinned()) vp.fold = fold_plan(n1, n2, n3, vp.hp);
     {  // shapes measured earlier for this size (this process or PK_TUNE_FILE)
         Wisdom& w = Wisdom::get();
         std::lock_guard<std::mutex> lk(w.mu);
@@ -650,7 +661,7 @@ constexpr float kTuneMargin = 0.03f;
 std::string pk_ctx_impl::autotune(int64_t n1, int64_t n2, int64_t n3) {
     const std::vector<int64_t> key{n1, n2, n3};
     const VolPlan& cur = plan(n1, n2, n3);
-    VolPlan vp = cur;
+    VolPlan vp = cur.three_pass();
     const int Lx = (int)(vp.packed ? n1 / 2 : n1);
     ensure(ws.A, sizeof(float2) * (size_t)vp.S);
     ensure(ws.I, sizeof(float) * (size_t)vp.N);
@@ -762,6 +773,31 @@ std::string pk_ctx_impl::autotune(int64_t n1, int64_t n2, int64_t n3) {
     std::snprintf(buf, sizeof buf, " | conv along dim %d (%.3f vs %.3f ms per transform pair)", vp.conv_axis,
                   std::min(order_y, order_z), std::max(order_y, order_z));
     rep += buf;
+    bool three = false;
+    // the two-pass form against the three-pass one: a half iteration of each (the built-in choice is the former)
+    if (const FoldPlan fp = tune().pinned() ? FoldPlan{} : fold_plan(n1, n2, n3, vp.hp); fp.on) {
+        auto half = [&](const VolPlan& t) {
+            return timed([&] {
+                const int oax = t.conv_axis == 3 ? 2 : 3;
+                if (!t.fold.on) run_col(t, oax, A, CM_FWD, nullptr, 1.f);
+                run_conv(t, A, H, false);
+                if (!t.fold.on) run_col(t, oax, A, CM_INV, nullptr, 1.f);
+                XArgs a{};
+                a.mode = XM_RATIO;
+                a.spec = A;
+                a.I = ws.I.as<float>();
+                run_x(t, a);
+            });
+        };
+        VolPlan two = vp;
+        two.fold = fp;
+        const float t3 = half(vp), t2 = half(two);
+        three = t3 < t2 * (1.f - kTuneMargin);
+        if (!three) vp = two;
+        std::snprintf(buf, sizeof buf, " | half iteration: three passes %.3f, two passes (%dx%d rows, T%d) %.3f ms", t3,
+                      fp.a, fp.b, fp.T, t2);
+        rep += buf;
+    }
     vp.tuned = true;
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
@@ -771,7 +807,8 @@ std::string pk_ctx_impl::autotune(int64_t n1, int64_t n2, int64_t n3) {
     {
         Wisdom& w = Wisdom::get();
         std::lock_guard<std::mutex> lk(w.mu);
-        w.store(key, {vp.x.fp.E, vp.y.fp.E, vp.y.nt, vp.y.tile, vp.z.fp.E, vp.z.nt, vp.z.tile, vp.conv_axis});
+        w.store(key, {three ? -vp.x.fp.E : vp.x.fp.E, vp.y.fp.E, vp.y.nt, vp.y.tile, vp.z.fp.E, vp.z.nt, vp.z.tile,
+                      vp.conv_axis});
     }
     std::snprintf(buf, sizeof buf, "%lldx%lldx%lld: x E%d; y E%d/%d/T%d; z E%d/%d/T%d; conv dim %d |",
                   (long long)n1, (long long)n2, (long long)n3, vp.x.fp.E, vp.y.fp.E, vp.y.nt, vp.y.tile, vp.z.fp.E,
@@ -830,6 +867,34 @@ void pk_ctx_impl::run_graphed(const std::vector<uint64_t>& key, Fn&& fn) {
 }
 
 // ------------------------------------------------------------------ passes
+void pk_ctx_impl::run_foldx(const VolPlan& vp, const XArgs& a, int64_t z0, int64_t nz) {
+    const FoldPlan& fp = vp.fold;
+    FoldX f = fp.x;
+    f.a = a;
+    f.tw = vp.x.fp.tw;
+    f.twy = vp.y.fp.tw;
+    f.blk0 = (int)(z0 * f.nyb);
+    PK_HIP(launch_foldx(fp.xnt, dim3((unsigned)(nz * f.nyb)), fp.xlds, stream, f, a.mode, nullptr, nullptr, 0));
+}
+
+void pk_ctx_impl::run_foldc(const VolPlan& vp, float2* data, int mode, const float2* otf) {
+    const FoldPlan& fp = vp.fold;
+    FoldC f = fp.c;
+    f.data = data;
+    f.otf = otf;
+    f.twy = vp.y.fp.tw;
+    f.twz = vp.z.fp.tw;
+    hipEvent_t e0 = prof_mark();
+    PK_HIP(launch_foldc(fp.cnt, dim3((unsigned)fp.cblocks), fp.clds, stream, f, mode, nullptr, nullptr, 0));
+    if (prof_on) prof_done(mode == CM_FWD ? "yz_fwd" : "yz_conv", (mode == CM_FWD ? 16.0 : 24.0) * (double)vp.Sa, e0);
+}
+
+void pk_ctx_impl::run_conv(const VolPlan& vp, float2* data, const float2* otf, bool conj) {
+    const int mode = conj ? CM_CONVJ : CM_CONV;
+    if (vp.fold.on) run_foldc(vp, data, mode, otf);
+    else run_col(vp, vp.conv_axis, data, mode, otf, (float)(1.0 / (double)vp.N));
+}
+
 void pk_ctx_impl::run_x(const VolPlan& vp, XArgs a, int64_t z0, int64_t nz) {
     a.n1 = (int)vp.n1;
     a.h1 = (int)vp.h1;
@@ -841,7 +906,7 @@ void pk_ctx_impl::run_x(const VolPlan& vp, XArgs a, int64_t z0, int64_t nz) {
     a.eps = kEps;
     if (nz <= 0) nz = vp.n3 - z0;
     a.nrows = vp.n2 * nz;
-    if (z0 > 0) {
+    if (z0 > 0 && !vp.fold.on) {
         // slab: every array advanced to plane z0; block partials continue the
         // whole-volume numbering (slab boundaries fall on block boundaries)
         const int64_t ro = z0 * vp.n2 * vp.n1;
@@ -868,7 +933,8 @@ void pk_ctx_impl::run_x(const VolPlan& vp, XArgs a, int64_t z0, int64_t nz) {
     hipEvent_t e0 = prof_mark();
     // compile-time kernel when one exists for this (row length, values per
     // thread) and the tile is the full 256-thread block it assumes
-    if (vp.x.block.x == (unsigned)kMaxThreads && !tune().generic_x &&
+    if (vp.fold.on) run_foldx(vp, a, z0, nz);
+    else if (vp.x.block.x == (unsigned)kMaxThreads && !tune().generic_x &&
         launch_xrow(vp.packed ? vp.x.fp.L : -vp.x.fp.L, vp.x.fp.E, dim3((unsigned)nblk), vp.x.lds, stream, a,
                     vp.x.fp.tw))
         PK_HIP(hipGetLastError());
@@ -906,7 +972,6 @@ void pk_ctx_impl::run_x(const VolPlan& vp, XArgs a, int64_t z0, int64_t nz) {
     }
 }
 
-static int64_t xpass_blocks(const VolPlan& vp) { return (vp.n2 * vp.n3 + vp.x.tile - 1) / vp.x.tile; }
 
 void pk_ctx_impl::run_col(const VolPlan& vp, int axis, float2* data, int mode, const float2* otf, float scale,
                           int64_t z0, int64_t nz) {
@@ -947,22 +1012,24 @@ void pk_ctx_impl::run_col(const VolPlan& vp, int axis, float2* data, int mode, c
     }
 }
 
-void pk_ctx_impl::r2c3d(const VolPlan& vp, const float* real, float2* spec) {
+void pk_ctx_impl::r2c3d(const VolPlan& plan_, const float* real, float2* spec) {
+    const VolPlan vp = plan_.three_pass();  // natural frequency order
     XArgs a{};
     a.mode = XM_R2C;
-        a.src = real;
+    a.src = real;
     a.spec = spec;
     run_x(vp, a);
     run_col(vp, 2, spec, CM_FWD, nullptr, 1.f);
     run_col(vp, 3, spec, CM_FWD, nullptr, 1.f);
 }
 
-void pk_ctx_impl::c2r3d(const VolPlan& vp, float2* spec, float* real) {
+void pk_ctx_impl::c2r3d(const VolPlan& plan_, float2* spec, float* real) {
+    const VolPlan vp = plan_.three_pass();
     run_col(vp, 3, spec, CM_INV, nullptr, 1.f);
     run_col(vp, 2, spec, CM_INV, nullptr, 1.f);
     XArgs a{};
     a.mode = XM_C2R;
-        a.spec = spec;
+    a.spec = spec;
     a.dst = real;
     run_x(vp, a);
 }
@@ -974,13 +1041,14 @@ static int grid_for(int64_t n) { return (int)std::min<int64_t>((n + 255) / 256, 
 // device's memory-side cache; 0 = whole volume.  A slab holds whole x-pass
 // blocks (nz * n2 a multiple of the rows per block).  PK_SLAB_PLANES overrides.
 bool pk_ctx_impl::x_compile_time(const VolPlan& vp) const {
-    return vp.x.block.x == (unsigned)kMaxThreads && !tune().generic_x &&
-           xrow_available(vp.packed ? vp.x.fp.L : -vp.x.fp.L, vp.x.fp.E);
+    return vp.fold.on || (vp.x.block.x == (unsigned)kMaxThreads && !tune().generic_x &&
+                          xrow_available(vp.packed ? vp.x.fp.L : -vp.x.fp.L, vp.x.fp.E));
 }
 
 int64_t pk_ctx_impl::slab_planes(const VolPlan& vp) const {
     int64_t k = tune().slab >= 0 ? tune().slab : 0;
     if (k <= 0 || k >= vp.n3 || vp.conv_axis != 3) return 0;
+    if (vp.fold.on) return k;  // whole planes are whole blocks of the fold row pass
     while (k < vp.n3 && (k * vp.n2) % vp.x.tile != 0) ++k;
     return k >= vp.n3 ? 0 : k;
 }
@@ -1032,7 +1100,7 @@ const float2* pk_ctx_impl::otf_for(const VolPlan& vp, const float* psf, const in
 const float2* pk_ctx_impl::otf_find(const VolPlan& vp, uint64_t h, const int64_t pd[3]) {
     for (auto& e : otf) {
         if (e.dims[0] == vp.n1 && e.dims[1] == vp.n2 && e.dims[2] == vp.n3 && e.hash == h &&
-            e.pdims[0] == pd[0] && e.pdims[1] == pd[1] && e.pdims[2] == pd[2]) {
+            e.layout == vp.fold.layout && e.pdims[0] == pd[0] && e.pdims[1] == pd[1] && e.pdims[2] == pd[2]) {
             e.tick = ++tick;
             return e.spec->as<float2>();
         }
@@ -1065,6 +1133,7 @@ const float2* pk_ctx_impl::otf_build(const VolPlan& vp, uint64_t h, const float*
     ent.dims[2] = vp.n3;
     std::memcpy(ent.pdims, pd, sizeof(int64_t) * 3);
     ent.hash = h;
+    ent.layout = vp.fold.layout;
     ent.tick = ++tick;
     ent.spec = std::make_unique<DevBuf>();
     alloc(*ent.spec, sizeof(float2) * (size_t)vp.S);
@@ -1104,7 +1173,16 @@ void pk_ctx_impl::build_otf_into(const VolPlan& vp, const float* q, const int64_
                            (int)pd[2], real, vp.n1, vp.n2, vp.n3);
         PK_HIP(hipGetLastError());
     }
-    r2c3d(vp, real, dst);
+    if (vp.fold.on) {  // in the order the fold passes read it
+        XArgs a{};
+        a.mode = XM_R2C;
+        a.src = real;
+        a.spec = dst;
+        run_x(vp, a);
+        run_foldc(vp, dst, CM_FWD, nullptr);
+    } else {
+        r2c3d(vp, real, dst);
+    }
 }
 
 void pk_ctx_impl::reset() {
@@ -1252,16 +1330,16 @@ void pk_ctx_impl::omw_passes(const VolPlan& vp, const XArgs& pa, float* I, float
                              const std::vector<uint64_t>* loop_key,
                              const std::function<void(int, const float*)>* after, uint16_t* I16) {
     const int64_t step = kz > 0 ? kz : vp.n3;
-    const float scale = (float)(1.0 / (double)vp.N);  // ifftn's 1/N
     auto slabs = [&](auto&& body) {
         for (int64_t z0 = 0; z0 < vp.n3; z0 += step) body(z0, std::min(step, vp.n3 - z0));
     };
     // the strided pass pair around the convolution (dim 2 unless the plan
     // convolves along dim 2); slabs only split dim-2 passes
     const int outer = vp.conv_axis == 3 ? 2 : 3;
-    auto y_fwd = [&](int64_t z0, int64_t nz) { run_col(vp, outer, A, CM_FWD, nullptr, 1.f, z0, nz); };
-    auto y_inv = [&](int64_t z0, int64_t nz) { run_col(vp, outer, A, CM_INV, nullptr, 1.f, z0, nz); };
-    auto z_conv = [&](const float2* H) { run_col(vp, vp.conv_axis, A, CM_CONV, H, scale); };
+    const bool fold = vp.fold.on;  // the row and convolution passes do the outer axis
+    auto y_fwd = [&](int64_t z0, int64_t nz) { if (!fold) run_col(vp, outer, A, CM_FWD, nullptr, 1.f, z0, nz); };
+    auto y_inv = [&](int64_t z0, int64_t nz) { if (!fold) run_col(vp, outer, A, CM_INV, nullptr, 1.f, z0, nz); };
+    auto z_conv = [&](const float2* H) { run_conv(vp, A, H, false); };
     slabs([&](int64_t z0, int64_t nz) {
         run_x(vp, pa, z0, nz);
         if (numit > 0) y_fwd(z0, nz);
@@ -1315,7 +1393,10 @@ void pk_ctx_impl::decon(int method, const pk_vol* Iv, const float* psf_f, const 
     const int64_t* od = g.od;
 
     if ((o->flags & PK_FLAG_AUTOTUNE) && !plan(n1, n2, n3).tuned) autotune(n1, n2, n3);
-    const VolPlan& vp = plan(n1, n2, n3);
+    const VolPlan& planned = plan(n1, n2, n3);
+    VolPlan natural;  // the unfused path's transforms are in natural order
+    if (o->flags & PK_FLAG_UNFUSED) natural = planned.three_pass();
+    const VolPlan& vp = (o->flags & PK_FLAG_UNFUSED) ? natural : planned;
     const int64_t N = vp.N;
     if (o->flags & PK_FLAG_NO_OTF_CACHE) {  // rebuild the OTFs on every call (comparison baseline)
         otf.erase(std::remove_if(otf.begin(), otf.end(), [](const OtfEntry& e) { return e.pins == 0; }), otf.end());
@@ -1327,7 +1408,7 @@ void pk_ctx_impl::decon(int method, const pk_vol* Iv, const float* psf_f, const 
     ensure(ws.I, sizeof(float) * N);
     ensure(ws.J, sizeof(float) * N);
     ensure(ws.A, sizeof(float2) * vp.S);
-    const int64_t nxb = xpass_blocks(vp);
+    const int64_t nxb = vp.x_blocks();
     if (method == 0) {
         ensure(ws.J3, sizeof(float) * N);
         ensure(ws.Y, sizeof(float) * N);
@@ -1414,16 +1495,14 @@ void pk_ctx_impl::decon(int method, const pk_vol* Iv, const float* psf_f, const 
         // its data from the memory-side cache; the dim-3 convolution covers the
         // whole volume between chains.  kz = 0: one slab (the whole volume).
         const int64_t step = kz > 0 ? kz : vp.n3;
-        const float scale = (float)(1.0 / (double)vp.N);  // ifftn's 1/N
         auto slabs = [&](auto&& body) {
             for (int64_t z0 = 0; z0 < vp.n3; z0 += step) body(z0, std::min(step, vp.n3 - z0));
         };
         const int outer = vp.conv_axis == 3 ? 2 : 3;
-        auto y_fwd = [&](int64_t z0, int64_t nz) { run_col(vp, outer, A, CM_FWD, nullptr, 1.f, z0, nz); };
-        auto y_inv = [&](int64_t z0, int64_t nz) { run_col(vp, outer, A, CM_INV, nullptr, 1.f, z0, nz); };
-        auto z_conv = [&](const float2* H, bool conj) {
-            run_col(vp, vp.conv_axis, A, conj ? CM_CONVJ : CM_CONV, H, scale);
-        };
+        const bool fold = vp.fold.on;
+        auto y_fwd = [&](int64_t z0, int64_t nz) { if (!fold) run_col(vp, outer, A, CM_FWD, nullptr, 1.f, z0, nz); };
+        auto y_inv = [&](int64_t z0, int64_t nz) { if (!fold) run_col(vp, outer, A, CM_INV, nullptr, 1.f, z0, nz); };
+        auto z_conv = [&](const float2* H, bool conj) { run_conv(vp, A, H, conj); };
 
         // the iteration loop reads only the workspace, the cached OTFs and the
         // plan's tables, so it is replayed as a graph for a repeated key

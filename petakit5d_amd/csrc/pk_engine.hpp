@@ -14,6 +14,7 @@
 
 #include "../../include/pkdecon.h"
 #include "pk_fft_dev.hpp"
+#include "pk_fold.hpp"
 
 namespace pk {
 
@@ -72,6 +73,15 @@ struct VolPlan {
     // forward pass before it and an inverse pass after it
     int conv_axis = 3;
     bool tuned = false;  // launch shapes and pass order measured by autotune()
+    FoldPlan fold;       // the two-pass form; off: the three passes above
+    // blocks of a row pass (the Biggs step length has one partial sum each)
+    int64_t x_blocks() const { return fold.on ? fold.xblocks : (n2 * n3 + x.tile - 1) / x.tile; }
+    // the same plan without the two-pass form (natural frequency order)
+    VolPlan three_pass() const {
+        VolPlan v = *this;
+        v.fold = FoldPlan{};
+        return v;
+    }
     // complex points of a row transform: n1 / 2 for packed (even) rows, n1 for odd rows
     int row_len() const { return (int)(packed ? n1 / 2 : n1); }
 };
@@ -87,6 +97,7 @@ struct OtfEntry {
     int64_t pdims[3];
     uint64_t hash;
     uint64_t tick;
+    uint64_t layout = 0;  // FoldPlan::layout of the plan it was built for (0: natural order)
     int pins = 0;  // volumes in flight that read this OTF: never evicted while > 0
     std::unique_ptr<DevBuf> spec;
 };
@@ -257,6 +268,11 @@ struct pk_ctx_impl {
     void c2r3d(const VolPlan& vp, float2* spec, float* real);
     // z0, nz: the planes [z0, z0 + nz) of dim 3 (a slab); nz = 0 means all
     void run_x(const VolPlan& vp, XArgs a, int64_t z0 = 0, int64_t nz = 0);
+    // fold row kernel for a.mode over the planes [z0, z0 + nz) (run_x's two-pass form)
+    void run_foldx(const VolPlan& vp, const XArgs& a, int64_t z0, int64_t nz);
+    void run_foldc(const VolPlan& vp, float2* data, int mode, const float2* otf);
+    // dim-2 forward, dim-3 forward x OTF/N, inverses: one fold pass, or the three strided passes' middle one
+    void run_conv(const VolPlan& vp, float2* data, const float2* otf, bool conj);
     void run_col(const VolPlan& vp, int axis, float2* data, int mode, const float2* otf, float scale, int64_t z0 = 0,
                  int64_t nz = 0);
     int64_t slab_planes(const VolPlan& vp) const;

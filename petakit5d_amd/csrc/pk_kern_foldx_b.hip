@@ -1,0 +1,16 @@
+// pk_kern_foldx_b.hip -- row kernels of the two-pass form (pk_fold_dev.hpp), modes XM_OMW_UPDATE, XM_OMW_UPDATE_U16;
+// the modes are split over several translation units so they compile in parallel.
+#include "pk_fold.hpp"
+
+namespace pk {
+bool launch_foldx_b(unsigned nt, dim3 grid, size_t lds, hipStream_t s, const FoldX& f, int mode,
+                    const FoldX* ch, const int64_t* starts, int n) {
+    switch (mode) {
+        case XM_OMW_UPDATE:
+            return launch_foldx_kernel(k_foldx<XM_OMW_UPDATE>, nt, grid, lds, s, f, ch, starts, n);
+        case XM_OMW_UPDATE_U16:
+            return launch_foldx_kernel(k_foldx<XM_OMW_UPDATE_U16>, nt, grid, lds, s, f, ch, starts, n);
+        default: return false;
+    }
+}
+}  // namespace pk

@@ -1,0 +1,100 @@
+"""The two-pass form of the iteration (pk_fold_dev.hpp) against the oracle and
+against the three-pass form, which pk_tune_set pins.
+
+Sizes cover its branches: one and two dim-2 steps in the row pass, one to
+three steps along the row, none and one dim-2 step in the column pass, one to
+three along dim 3, 8- and 16-column tiles, tiles whose last columns are padding,
+one and two row groups per block.  No other test uses these sizes: a pinned
+size stays pinned for the process's later plans."""
+import numpy as np
+import pytest
+
+import petakit5d_amd as pk
+from petakit5d_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [
+    (64, 32, 50),    # two row groups per block, one dim-2 step between the rows
+    (54, 120, 36),   # rows of 27 pairs, two dim-2 steps
+    (60, 48, 30),
+    (96, 135, 20),   # odd dim 2
+    (128, 36, 45),
+    (250, 40, 27),   # three steps of 5 along the row
+    (640, 16, 18),   # the smallest dim-2 step
+    (30, 540, 16),   # one step along the row, one along dim 3
+    (90, 16, 243),   # dim 2 whole in the row pass, three steps along dim 3
+    (50, 64, 32),
+    (72, 64, 16),
+    (54, 1024, 100),  # the largest dim-2 steps, 8-column tiles
+]
+
+
+def _volume(shape, seed):
+    g = np.random.default_rng(seed)
+    psf = synth.gaussian_psf(tuple(min(n, 9) for n in shape), 1.2, 2.0, 10.0)
+    img = synth._fft_convolve_circular(synth.point_emitters(shape, 60, (500, 3000), g), psf) + 100
+    return synth.poisson_u16(img, g), psf, np.ascontiguousarray(psf[::-1, ::-1, ::-1])
+
+
+def _rel(a, b):
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    return float(np.linalg.norm(a - b) / np.linalg.norm(b))
+
+
+def _three_pass(shape):
+    """A context whose plan of this size is pinned to the three-pass kernels."""
+    ctx = pk.Context(0)
+    L = shape[0] // 2
+    divisors = [1, 2, 3, 4, 5, 6, 8, 9, 10, 12, 15, 16, 18, 20, 24, 25, 27, 30, 32]
+
+    def cover(n, tile):
+        """Values per thread of an all-register plan of n points whose tile fits a 256-thread block."""
+        for e in divisors:
+            if n % e == 0 and n // e * tile <= 256 and all(e % p == 0 for p in (2, 3, 5) if n % p == 0):
+                return e
+        return None
+
+    def axis(n):
+        for tile in (16, 8, 4, 2, 1):
+            if cover(n, tile):
+                return cover(n, tile), 256, tile
+        raise AssertionError(n)
+
+    ctx.tune_set(shape, (cover(L, 1),) + axis(shape[1]) + axis(shape[2]) + (3,))
+    return ctx
+
+
+@pytest.mark.parametrize("shape", SIZES, ids=lambda s: "x".join(map(str, s)))
+def test_two_pass_form_matches_oracle_and_three_pass(oracle, shape):
+    I, psf, psf_b = _volume(shape, sum(shape))
+    two = pk.Context(0)  # before the pin: plans made later in the process take it
+    J2 = pk.decon_lucy_omw_function(I, psf, psf_b, 2, Background=100, save16bit=False, ctx=two)[0]
+    R2 = pk.decon_lucy_function(I.astype(np.float32), psf, 4, Background=100, save16bit=False, ctx=two)[0]
+    O2 = oracle.decon_lucy_omw_function(I, psf, psf_b, 2, Background=100, save16bit=False)[0]
+    OR = oracle.decon_lucy_function(I, psf, 4, Background=100, save16bit=False)[0]
+    # 32-bit sums over the transforms: the three-pass form is 2e-7 to 1.4e-6 from 64 bits on such volumes; a wrong
+    # index, twiddle or element is off by 1e-3 or more
+    assert _rel(J2, O2) <= 1e-5
+    assert _rel(R2, OR) <= 1e-5
+    three = _three_pass(shape)
+    J3 = pk.decon_lucy_omw_function(I, psf, psf_b, 2, Background=100, save16bit=False, ctx=three)[0]
+    R3 = pk.decon_lucy_function(I.astype(np.float32), psf, 4, Background=100, save16bit=False, ctx=three)[0]
+    assert _rel(J2, J3) <= 1e-5
+    assert _rel(R2, R3) <= 1e-5
+
+
+def test_two_pass_batch_and_options_equal_single_calls():
+    """Chunks of several sizes (padded ones among them) in one call give the single calls' bits; so do the options that
+    ride in the last update."""
+    shapes = [(60, 60, 30), (80, 64, 45), (53, 40, 27), (96, 64, 32), (45, 40, 27)]
+    vols = [_volume(s, 7 + k)[0] for k, s in enumerate(shapes)]
+    _, psf, psf_b = _volume((32, 32, 24), 1)
+    for method, it in (("omw", 2), ("rl", 4)):
+        for kw in ({}, {"dampFactor": 2, "scaleFactor": 0.5, "deconOffset": 3}, {"save16bit": False}):
+            outs = pk.decon_batch(vols, psf, psf_b, it, method=method, Background=100, **kw)
+            for v, o in zip(vols, outs):
+                args = (psf, psf_b, it) if method == "omw" else (psf, it)
+                fn = pk.decon_lucy_omw_function if method == "omw" else pk.decon_lucy_function
+                J = fn(v, *args, Background=100, pad=True, **kw)[0]
+                assert np.array_equal(o, J), (method, kw, v.shape)

@@ -114,7 +114,7 @@ def edge_erosion_mask(im, EdgeErosion, ctx=None):
         vm = PkVol(ctypes.c_void_p(m.data_ptr()), PK_UINT8, PK_MEM_DEVICE, (ctypes.c_int64 * 3)(*shape))
         torch.cuda.current_stream(t.device).synchronize()
         ctx.check(_lib.load().pk_edge_erosion_mask(ctx.handle, ctypes.byref(vin), int(EdgeErosion), ctypes.byref(vm)))
-        return m.bool()
+        return m.view(torch.bool)  # 0 / 1 bytes
     a = np.asarray(im.numpy() if _is_torch(im) else im)
     if a.dtype not in (np.uint16, np.float32):
         a = a.astype(np.float32)

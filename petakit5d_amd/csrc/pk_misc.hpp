@@ -147,6 +147,19 @@ __global__ void k_edt_mask_pass1(const uint16_t* __restrict__ raw16, const float
 __global__ void k_edt_mask_pass(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst, int64_t n1, int64_t n2,
                                 int64_t n3, int axis, int R);
 __global__ void k_edt_mask_final(const uint16_t* __restrict__ d, uint8_t* __restrict__ mask, int64_t n, int R);
+// the same for R <= kBallMaxR and n1 <= 4096, on bits: false voxels as bits along dim 1 (W words a row), then the ball
+constexpr int kBallMaxR = 23;
+constexpr int kBallRows = 1653;  // integer points of the disk of radius kBallMaxR
+struct BallRows {                // rows (dx, dz) in order of falling half-width h; those of h end at end[h]
+    int R;
+    int16_t end[kBallMaxR + 1];
+    int8_t dx[kBallRows], dz[kBallRows];
+};
+BallRows ball_rows(int R);
+__global__ void k_false_bits(const uint16_t* __restrict__ raw16, const float* __restrict__ rawf, int64_t n1, int64_t n2,
+                             int64_t n3, int W, unsigned long long* __restrict__ bits);
+__global__ void k_ball_mask(const unsigned long long* __restrict__ bits, int64_t n1, int64_t n2, int64_t n3, int W,
+                            BallRows ball, uint8_t* __restrict__ mask);
 __global__ void k_mask_erode_z(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, int64_t n1, int64_t n2,
                                int64_t n3, int h, const unsigned long long* __restrict__ count);
 

@@ -412,6 +412,14 @@ pk_status pk_deskew_rotate_frame3d_resample(pk_ctx *ctx, const pk_vol *in, doubl
                                             double x_step_thresh, const double resample[3], int32_t interp,
                                             const int64_t bbox[6], pk_vol *out);
 
+/* The extents rotateFrame3D.m:46-66 takes from proj = squeeze(max(vol, [], 1))'
+ * ~= 0 of the column-major device volume d_vol: over the points (x, z), 1-based,
+ * of find(diff(proj, 1, 2)), c = s x + k z zx_ratio and cx = k x - s z zx_ratio
+ * with s = sin_theta, k = cos_theta.  out = {1 if there is such a point else 0,
+ * min c, max c, min cx, max cx} (host; inf and -inf when there is none). */
+pk_status pk_rotate_extent(pk_ctx *ctx, const float *d_vol, const int64_t dims[3], double sin_theta, double cos_theta,
+                           double zx_ratio, double out[5]);
+
 /* Affine resampling as imwarp(vol, affine3d(T), 'linear', 'FillValues', 0,
  * 'OutputView', imref3d(out_dims, 1, 1, 1)) does for rotateFrame3D
  * (pointDetection/llsmtools/transforms/rotateFrame3D.m:46-100, used after

@@ -83,6 +83,7 @@ EXPORTS = [
     "pk_deskew_rotate_out_dims",
     "pk_deskew_rotate_frame3d",
     "pk_affine_warp3d",
+    "pk_rotate_extent",
 ]
 
 

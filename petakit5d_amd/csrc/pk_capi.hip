@@ -383,6 +383,16 @@ pk_status pk_edge_erosion_mask(pk_ctx* c, const pk_vol* im, int32_t edge_erosion
     return guarded(c, [&] { c->edge_erosion_mask(im, edge_erosion, mask); });
 }
 
+pk_status pk_rotate_extent(pk_ctx* c, const float* d_vol, const int64_t dims[3], double sin_theta, double cos_theta,
+                           double zx_ratio, double out[5]) {
+    return guarded(c, [&] {
+        if (!d_vol || !dims || !out) pk::fail(PK_ERR_INVALID_ARG, "null argument");
+        for (int i = 0; i < 3; ++i)
+            if (dims[i] < 1) pk::fail(PK_ERR_INVALID_ARG, "volume dimensions must be >= 1");
+        c->edge_extents(d_vol, dims, sin_theta, cos_theta, zx_ratio, out);
+    });
+}
+
 pk_status pk_affine_warp3d(pk_ctx* c, const float* d_vol, const int64_t dims[3], const double inv_tform[16],
                            const int64_t out_dims[3], float* d_out) {
     return guarded(c, [&] {

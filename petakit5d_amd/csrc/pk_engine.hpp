@@ -329,6 +329,8 @@ struct pk_ctx_impl {
     void deskew_rotate(const pk_vol* in, double angle, double dz, double xy, bool reverse, bool objective,
                        double x_step_thresh, const int64_t* bbox, pk_vol* out, int interp = 0,
                        const double* rs = nullptr, bool imwarp_form = false);
+    // {any, min c, max c, min cx, max cx} of rotateFrame3D.m:46-66 over the edges of max(vol, [], 1) ~= 0 (pk_deskew.hip)
+    void edge_extents(const float* vol, const int64_t dims[3], double a, double b, double zx, double out[5]);
     // bwdist(~bw) > E - 1 of bw = im > 0 with cleared faces (RLdecon_large_in_memory.m:150-155)
     void edge_erosion_mask(const pk_vol* im, int E, pk_vol* mask);
     // copy of a pitched half spectrum with one pass's access pattern (pk_probe.hip): ms per copy

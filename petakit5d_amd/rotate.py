@@ -28,28 +28,35 @@ def _translate(t):
 
 
 def rotate_transform(shape, angle, zxRatio, reverse=False, Crop=True, resample=None, ObjectiveScan=False,
-                     outSize=None, proj=None):
+                     outSize=None, proj=None, extents=None):
     """(T, outSize) of rotateFrame3D for a volume of MATLAB size shape: T the
     4x4 forward transform in imwarp's row-vector convention ([x y z 1] * T),
     outSize [ny' nx' nz'].  proj: the volume's max over dim 1 as an nx x nz
-    array (needed for the crop decision of stage scans)."""
+    array (needed for the crop decision of stage scans), or extents(a, b): the
+    same projection's (any, min c, max c, min cx, max cx) from the device."""
     ny, nx, nz = (int(n) for n in shape)
     theta = angle * math.pi / 180
     if reverse:
         theta = -theta
     do_crop, w, h = False, None, None
     if not ObjectiveScan:  # rotateFrame3D.m:46-66
-        pz = (np.asarray(proj) != 0).T.astype(np.int8)  # squeeze(max(vol, [], 1))' ~= 0: nz x nx
-        d = np.diff(pz, axis=1)  # diff(proj, 1, 2)
-        xs, zs = np.nonzero(d.T)  # [z, x] = find(proj ~= 0), in find's column-major order
-        z, x = zs + 1.0, xs + 1.0
         a, b = math.sin(-theta), math.cos(-theta)
-        if z.size:
-            c = a * x + b * z * zxRatio
-            h = _mround(c.max() - c.min()) - 4
+        if extents is not None:
+            found, c0, c1, cx0, cx1 = extents(a, b)
+        else:
+            pz = (np.asarray(proj) != 0).T.astype(np.int8)  # squeeze(max(vol, [], 1))' ~= 0: nz x nx
+            d = np.diff(pz, axis=1)  # diff(proj, 1, 2)
+            xs, zs = np.nonzero(d.T)  # [z, x] = find(proj ~= 0), in find's column-major order
+            z, x = zs + 1.0, xs + 1.0
+            found = z.size
+            if found:
+                c = a * x + b * z * zxRatio
+                cx = b * x + (-a) * z * zxRatio
+                c0, c1, cx0, cx1 = c.min(), c.max(), cx.min(), cx.max()
+        if found:
+            h = _mround(c1 - c0) - 4
             do_crop = h < max(abs(a * (nx - 1) + b * (nz - 1) * zxRatio), abs(a * (nx - 1) + b * (1 - nz) * zxRatio))
-            cx = b * x + (-a) * z * zxRatio
-            w = _mround(cx.max() - cx.min()) - 4
+            w = _mround(cx1 - cx0) - 4
     center = np.array([ny, nx, nz], dtype=np.float64) + 1
     center /= 2
     T1 = _translate(-center[[1, 0, 2]])
@@ -100,14 +107,20 @@ def rotateFrame3D(vol, angle, zxRatio, reverse=False, Crop=True, resample=None, 
     d = tuple(int(n) for n in t.shape)
     if t.stride() != (1, d[0], d[0] * d[1]):
         t = t.permute(2, 1, 0).contiguous().permute(2, 1, 0)
-    proj = None if ObjectiveScan else t.amax(dim=0).cpu().numpy()
-    T, od = rotate_transform(d, angle, zxRatio, reverse, Crop, resample, ObjectiveScan, outSize, proj)
+    ctx = ctx or _lib.default_context()
+    torch.cuda.current_stream(t.device).synchronize()
+
+    def extents(a, b):  # of max(vol, [], 1) ~= 0, on the device
+        e = (ctypes.c_double * 5)()
+        ctx.check(_lib.load().pk_rotate_extent(ctx.handle, ctypes.c_void_p(t.data_ptr()), i64x3(d), ctypes.c_double(a),
+                                               ctypes.c_double(b), ctypes.c_double(zxRatio), e))
+        return tuple(e)
+
+    T, od = rotate_transform(d, angle, zxRatio, reverse, Crop, resample, ObjectiveScan, outSize, extents=extents)
     if min(od) < 1:
         raise ValueError(f"rotateFrame3D: output size {od}")
     inv = np.ascontiguousarray(np.linalg.inv(T), dtype=np.float64)
     out = torch.empty((od[2], od[1], od[0]), dtype=torch.float32, device=t.device).permute(2, 1, 0)
-    ctx = ctx or _lib.default_context()
-    torch.cuda.current_stream(t.device).synchronize()
     fn = _lib.load().pk_affine_warp3d_cubic if interp == "cubic" else _lib.load().pk_affine_warp3d
     ctx.check(fn(ctx.handle, ctypes.c_void_p(t.data_ptr()), i64x3(d), inv.ctypes.data_as(ctypes.POINTER(ctypes.c_double)),
                  i64x3(od), ctypes.c_void_p(out.data_ptr())))

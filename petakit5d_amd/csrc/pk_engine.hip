@@ -1666,11 +1666,28 @@ void pk_ctx_impl::edge_erosion_mask(const pk_vol* im, int E, pk_vol* mask) {
         const int W = (int)((n1 + 63) / 64);
         const int64_t rows = n2 * n3;
         unsigned long long* bits = ws.tmp.as<unsigned long long>();
-        const int64_t groups = (rows + 64 / W - 1) / (64 / W);
-        hipLaunchKernelGGL(k_false_bits, dim3((unsigned)std::min<int64_t>((rows + 3) / 4, 65536)), dim3(256), 0, stream,
-                           r16, rf, n1, n2, n3, W, bits);
-        hipLaunchKernelGGL(k_ball_mask, dim3((unsigned)std::min<int64_t>((groups + 3) / 4, 65536)), dim3(256), 0,
-                           stream, bits, n1, n2, n3, W, ball_rows(R), m);
+        if (n1 % 8 == 0 && reinterpret_cast<uintptr_t>(raw) % 16 == 0 && rows * W < (1 << 28)) {
+            const int64_t blocks = (rows * W * 8 + 1023) / 1024;
+            hipLaunchKernelGGL(k_false_bytes, dim3((unsigned)std::min<int64_t>(blocks, 1 << 20)), dim3(256), 0, stream,
+                               r16, rf, (uint32_t)n1, (uint32_t)n2, (uint32_t)n3, (uint32_t)W,
+                               reinterpret_cast<uint8_t*>(bits));
+        } else {
+            hipLaunchKernelGGL(k_false_bits, dim3((unsigned)std::min<int64_t>((rows + 3) / 4, 65536)), dim3(256), 0,
+                               stream, r16, rf, n1, n2, n3, W, bits);
+        }
+        // the tile where two blocks' tiles fit a CU's LDS
+        const int tx = 4 * (64 / W);
+        const size_t lds = (size_t)(tx + 2 * R) * (kBallTz + 2 * R) * W * 8;
+        const int64_t tiles = ((n2 + tx - 1) / tx) * ((n3 + kBallTz - 1) / kBallTz);
+        if (lds <= kMaxLds / 2 && tiles <= 0xFFFFFF) {
+            if (lds > 65536) allow_large_lds(k_ball_tile);
+            hipLaunchKernelGGL(k_ball_tile, dim3((unsigned)tiles), dim3(256), lds, stream, bits, n1, (int)n2, (int)n3,
+                               W, ball_rows(R), m);
+        } else {
+            const int64_t groups = (rows + 64 / W - 1) / (64 / W);
+            hipLaunchKernelGGL(k_ball_mask, dim3((unsigned)std::min<int64_t>((groups + 3) / 4, 65536)), dim3(256), 0,
+                               stream, bits, n1, n2, n3, W, ball_rows(R), m);
+        }
         PK_HIP(hipGetLastError());
         if (mask->mem == PK_MEM_HOST)
             PK_HIP(hipMemcpyAsync(mask->data, m, (size_t)N, hipMemcpyDeviceToHost, stream));

@@ -156,6 +156,11 @@ struct BallRows {                // rows (dx, dz) in order of falling half-width
     int8_t dx[kBallRows], dz[kBallRows];
 };
 BallRows ball_rows(int R);
+constexpr int kBallTz = 8;  // z rows of a thread of k_ball_tile
+__global__ void k_false_bytes(const uint16_t* __restrict__ raw16, const float* __restrict__ rawf, uint32_t n1,
+                              uint32_t n2, uint32_t n3, uint32_t W, uint8_t* __restrict__ bits);
+__global__ void k_ball_tile(const unsigned long long* __restrict__ bits, int64_t n1, int n2, int n3, int W,
+                            BallRows ball, uint8_t* __restrict__ mask);
 __global__ void k_false_bits(const uint16_t* __restrict__ raw16, const float* __restrict__ rawf, int64_t n1, int64_t n2,
                              int64_t n3, int W, unsigned long long* __restrict__ bits);
 __global__ void k_ball_mask(const unsigned long long* __restrict__ bits, int64_t n1, int64_t n2, int64_t n3, int W,

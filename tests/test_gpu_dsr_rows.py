@@ -1,7 +1,7 @@
-"""The row kernel of deskewRotateFrame3D at its edges: four values a lane and
-one value a lane give the same bits (a window that starts off a multiple of
-four rows takes the second), for one and two chunks of dim 1, runs of y that
-are cut short and windows of a few columns; against the oracle as well."""
+"""The row kernel of deskewRotateFrame3D at its edges: eight, four and one value
+a lane give the same bits (a window that starts off a multiple of eight or four
+rows takes the narrower), for one and two chunks of dim 1, runs of y that are
+cut short and windows of a few columns; against the oracle as well."""
 import numpy as np
 import pytest
 
@@ -10,7 +10,7 @@ import deskew_oracle as D
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("shape", [(64, 40, 12), (260, 33, 9), (67, 25, 14)])
+@pytest.mark.parametrize("shape", [(64, 40, 12), (260, 33, 9), (264, 33, 9), (67, 25, 14)])
 @pytest.mark.parametrize("dz,reverse", [(0.2, False), (0.3, True), (0.5, False), (0.5, True)])
 @pytest.mark.parametrize("u16", [False, True])
 def test_windows_equal_the_whole(shape, dz, reverse, u16):

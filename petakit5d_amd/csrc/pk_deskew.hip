@@ -14,14 +14,17 @@
 //
 // MATLAB volumes are column-major: a column (fixed x, z) is ny contiguous
 // floats, and every value of an output column uses the same two input columns
-// and weight.  One block per output column computes the source position once
-// and walks down the column: coalesced reads and writes, HBM-bound (4 bytes
-// read + 4 written per value; the second input column comes from cache).
+// and weight.  A block takes eight neighbouring output columns: they read nine
+// neighbouring input columns, each once.  Coalesced and HBM-bound (4 bytes read
+// + 4 written per value).  512x512x256 at 31.5 degrees, dz 0.2, pixel 0.108: 0.140 ms; with a
+// block per output column 0.172 ms (both columns of a blend read by every block:
+// 512 instead of 268 MB past L2).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <type_traits>
 
 #include "pk_engine.hpp"
 
@@ -54,42 +57,65 @@ DeskewGeom deskew_geometry(const int64_t dims[3], double angle, double dz, doubl
 
 // VEC: ny % 4 == 0 and 16-byte aligned buffers, so every column is whole
 // float4s (one 16-byte load per operand and one store per four values).
+constexpr int kDeskewRun = 8;
 template <bool VEC>
 __global__ void __launch_bounds__(256) k_deskew(const float* __restrict__ vol, float* __restrict__ out, int64_t ny,
-                                                int64_t nx, int64_t nx_out, double xstep, double xshift) {
-    // one block per output column (c, p); its threads walk down the column
-    const int64_t col = blockIdx.x;
-    const int64_t c = col % nx_out, p = col / nx_out;
-    const double x = (double)(c + 1) - xstep * (double)(p + 1) - xshift;  // 1-based input column
-    float* __restrict__ o = out + col * ny;
-    if (!(x >= 0.0 && x <= (double)(nx + 1))) {
-        if constexpr (VEC) {
-            for (int64_t r = threadIdx.x; r < ny / 4; r += blockDim.x)
-                reinterpret_cast<float4*>(o)[r] = make_float4(0.f, 0.f, 0.f, 0.f);
-        } else {
-            for (int64_t r = threadIdx.x; r < ny; r += blockDim.x) o[r] = 0.f;
-        }
-        return;
+                                                int64_t nx, int64_t nx_out, double xstep, double xshift, uint32_t runs,
+                                                uint32_t total, uint32_t per_xcd) {
+    using V = std::conditional_t<VEC, float4, float>;
+    // one block per run of kDeskewRun output columns of a plane; its threads
+    // walk down the columns.  Blocks go round-robin to the 8 XCDs: each XCD
+    // walks a contiguous range
+    const uint32_t item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (item >= total) return;
+    const int64_t p = item / runs, c0 = (int64_t)(item - (uint32_t)p * runs) * kDeskewRun;
+    const int n = (int)(nx_out - c0 < kDeskewRun ? nx_out - c0 : kDeskewRun);
+    const int64_t rows = VEC ? ny / 4 : ny;
+    auto zero = [] {
+        if constexpr (VEC) return make_float4(0.f, 0.f, 0.f, 0.f);
+        else return 0.f;
+    };
+    auto blend = [](const V& a, const V& b, float f) {
+        if constexpr (VEC)
+            return make_float4(a.x + f * (b.x - a.x), a.y + f * (b.y - a.y), a.z + f * (b.z - a.z),
+                               a.w + f * (b.w - a.w));
+        else return a + f * (b - a);
+    };
+    // 1-based input column of every output column; outside [0, nx + 1]: 0s
+    int64_t i0[kDeskewRun];
+    float f[kDeskewRun];
+    bool any = false, row = n == kDeskewRun;  // row: neighbours read neighbours
+#pragma unroll
+    for (int k = 0; k < kDeskewRun; ++k) {
+        const double x = (double)(c0 + k + 1) - xstep * (double)(p + 1) - xshift;
+        const bool in = k < n && x >= 0.0 && x <= (double)(nx + 1);
+        const double x0 = std::floor(in ? x : -1.0);
+        i0[k] = (int64_t)x0;  // 0 ... nx + 1, or -1
+        f[k] = in ? (float)(x - x0) : 0.f;
+        any |= in;
+        row = row && in && (k == 0 || i0[k] == i0[k > 0 ? k - 1 : 0] + 1);
     }
-    const double x0 = std::floor(x);
-    const float f = (float)(x - x0);
-    const int64_t i0 = (int64_t)x0;  // 0 ... nx + 1
-    const float* __restrict__ plane = vol + p * ny * nx;
-    const float* __restrict__ ca = (i0 >= 1 && i0 <= nx) ? plane + (i0 - 1) * ny : nullptr;
-    const float* __restrict__ cb = (i0 + 1 >= 1 && i0 + 1 <= nx) ? plane + i0 * ny : nullptr;
-    if constexpr (VEC) {
-        const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int64_t r = threadIdx.x; r < ny / 4; r += blockDim.x) {
-            const float4 a = ca ? reinterpret_cast<const float4*>(ca)[r] : z;
-            const float4 b = cb ? reinterpret_cast<const float4*>(cb)[r] : z;
-            reinterpret_cast<float4*>(o)[r] =
-                make_float4(a.x + f * (b.x - a.x), a.y + f * (b.y - a.y), a.z + f * (b.z - a.z), a.w + f * (b.w - a.w));
-        }
-    } else {
-        for (int64_t r = threadIdx.x; r < ny; r += blockDim.x) {
-            const float a = ca ? ca[r] : 0.f;
-            const float b = cb ? cb[r] : 0.f;
-            o[r] = a + f * (b - a);
+    V* __restrict__ o = reinterpret_cast<V*>(out + (p * nx_out + c0) * ny);
+    const V* __restrict__ src = reinterpret_cast<const V*>(vol + p * ny * nx);
+    auto col = [&](int64_t i, int64_t r) { return i >= 1 && i <= nx ? src[(i - 1) * rows + r] : zero(); };
+    for (int64_t r = threadIdx.x; r < rows; r += blockDim.x) {
+        if (row) {
+            V v[kDeskewRun + 1];
+#pragma unroll
+            for (int k = 0; k <= kDeskewRun; ++k) v[k] = col(i0[0] + k, r);
+#pragma unroll
+            for (int k = 0; k < kDeskewRun; ++k) o[k * rows + r] = blend(v[k], v[k + 1], f[k]);
+        } else {
+            for (int k = 0; k < n; ++k) {
+                const double x = (double)(c0 + k + 1) - xstep * (double)(p + 1) - xshift;
+                if (!any || !(x >= 0.0 && x <= (double)(nx + 1))) {
+                    o[k * rows + r] = zero();
+                    continue;
+                }
+                const double x0 = std::floor(x);
+                const int64_t i = (int64_t)x0;
+                o[k * rows + r] = blend(col(i, r), col(i + 1, r), (float)(x - x0));
+            }
         }
     }
 }
@@ -103,12 +129,13 @@ void launch_deskew(const float* vol, float* out, const int64_t dims[3], const De
     const unsigned nt = per_col >= 256 ? 256u : (unsigned)((per_col + 63) / 64 * 64);
     // the dispatch's grid size counts work-items in 32 bits
     if (cols * (int64_t)nt > 0xFFFFFFFFll) fail(PK_ERR_UNSUPPORTED_SIZE, "deskewed volume has too many columns");
-    if (vec)
-        hipLaunchKernelGGL(k_deskew<true>, dim3((unsigned)cols), dim3(nt), 0, s, vol, out, dims[0], dims[1], g.nx_out,
-                           g.xstep, g.xshift);
-    else
-        hipLaunchKernelGGL(k_deskew<false>, dim3((unsigned)cols), dim3(nt), 0, s, vol, out, dims[0], dims[1],
-                           g.nx_out, g.xstep, g.xshift);
+    const int64_t runs = (g.nx_out + kDeskewRun - 1) / kDeskewRun, total = runs * dims[2], per_xcd = (total + 7) / 8;
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(per_xcd * 8)), dim3(nt), 0, s, vol, out, dims[0], dims[1], g.nx_out,
+                           g.xstep, g.xshift, (uint32_t)runs, (uint32_t)total, (uint32_t)per_xcd);
+    };
+    if (vec) go(k_deskew<true>);
+    else go(k_deskew<false>);
     PK_HIP(hipGetLastError());
 }
 
@@ -169,8 +196,9 @@ __global__ void __launch_bounds__(256) k_affine3d(const float* __restrict__ vol,
 // wavefront takes 64 V values of kRowsRun neighbouring output columns of one
 // page; the wavefronts of a block take neighbouring pages and blocks go to the
 // XCDs in contiguous ranges, so that the input columns they share meet in L1
-// and L2.  Bound by the columns' reads from cache and the result's write:
-// 512x980x200 rotated by 31.5 degrees 0.181 ms, with the general kernel 0.311 ms.
+// and L2.  Bound by memory: 512x980x200 rotated by 31.5 degrees 0.180 ms (4.1
+// TB/s of the input read once and the result written), with the general kernel
+// 0.311 ms.
 constexpr int kRowsRun = 8;
 template <int V>
 __global__ void __launch_bounds__(256) k_affine_rows(const float* __restrict__ vol, float* __restrict__ out, int64_t ny,
@@ -235,30 +263,49 @@ __global__ void __launch_bounds__(256) k_affine_rows(const float* __restrict__ v
 // rotateFrame3D.m:46-66's extents without the projection leaving the device:
 // flag of a column = max over dim 1 ~= 0 (a positive value or a NaN settles it;
 // else true when no value is 0), one wavefront a column.  Bound by reading the
-// columns that hold only zeros.  512x980x200: 0.112 ms and 0.009 ms for the
+// columns that hold only zeros.  512x980x200: 0.076 ms and 0.009 ms for the
 // extents; the maximum as a reduction of the library, its copy and the host's
 // search were 0.6 ms.
+// A wavefront follows kFlagCols columns at once, 64 V values of each a step.
+constexpr int kFlagCols = 4;
+template <int V>
 __global__ void __launch_bounds__(256) k_column_flags(const float* __restrict__ vol, int64_t ny, int64_t cols,
                                                       uint8_t* __restrict__ flag) {
     const int ln = threadIdx.x & 63;
-    for (int64_t c = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); c < cols; c += (int64_t)gridDim.x * 4) {
-        const float* __restrict__ v = vol + c * ny;
-        bool settled = false, zero = false;
-        for (int64_t y = 0; y < ny && !settled; y += 256) {
-            bool pos = false;
+    const int64_t groups = (cols + kFlagCols - 1) / kFlagCols, step = (int64_t)gridDim.x * 4;
+    for (int64_t g = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); g < groups; g += step) {
+        const float* __restrict__ v = vol + g * kFlagCols * ny;
+        bool settled[kFlagCols], zero[kFlagCols] = {};
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int64_t i = y + k * 64 + ln;
+        for (int c = 0; c < kFlagCols; ++c) settled[c] = g * kFlagCols + c >= cols;
+        for (int64_t y = 0; y < ny; y += 64 * V) {
+            const int64_t i = y + (int64_t)ln * V;
+            float4 a[kFlagCols];
+            bool left = false;
+#pragma unroll
+            for (int c = 0; c < kFlagCols; ++c) {
+                a[c] = make_float4(-1.f, -1.f, -1.f, -1.f);  // neither positive nor 0
+                if (settled[c]) continue;
+                left = true;
                 if (i < ny) {
-                    const float a = v[i];
-                    pos |= !(a <= 0.f);
-                    zero |= a == 0.f;
+                    if constexpr (V == 4) a[c] = *reinterpret_cast<const float4*>(v + c * ny + i);
+                    else a[c].x = v[c * ny + i];
                 }
             }
-            settled = __ballot(pos) != 0;
+            if (!left) break;
+#pragma unroll
+            for (int c = 0; c < kFlagCols; ++c) {
+                if (settled[c]) continue;
+                const float4 t = a[c];
+                zero[c] |= t.x == 0.f || t.y == 0.f || t.z == 0.f || t.w == 0.f;
+                settled[c] = __ballot(!(t.x <= 0.f) || !(t.y <= 0.f) || !(t.z <= 0.f) || !(t.w <= 0.f)) != 0;
+            }
         }
-        const bool any_zero = __ballot(zero) != 0;
-        if (ln == 0) flag[c] = settled || !any_zero;
+#pragma unroll
+        for (int c = 0; c < kFlagCols; ++c) {
+            const bool any_zero = __ballot(zero[c]) != 0;
+            if (ln == 0 && g * kFlagCols + c < cols) flag[g * kFlagCols + c] = settled[c] || !any_zero;
+        }
     }
 }
 // Per block: whether a flag changes between columns x and x + 1 of a page
@@ -310,8 +357,12 @@ void pk_ctx_impl::edge_extents(const float* vol, const int64_t dims[3], double a
     ensure(ws.dsr, off + sizeof(double) * 5 * kBlocks);
     uint8_t* flag = ws.dsr.as<uint8_t>();
     double* part = reinterpret_cast<double*>(ws.dsr.as<char>() + off);
-    hipLaunchKernelGGL(k_column_flags, dim3((unsigned)std::min<int64_t>((cols + 3) / 4, 65536)), dim3(256), 0, stream,
-                       vol, dims[0], cols, flag);
+    const int64_t groups = (cols + kFlagCols - 1) / kFlagCols;
+    const dim3 grid((unsigned)std::min<int64_t>((groups + 3) / 4, 65536));
+    if (dims[0] % 4 == 0 && reinterpret_cast<uintptr_t>(vol) % 16 == 0)
+        hipLaunchKernelGGL(k_column_flags<4>, grid, dim3(256), 0, stream, vol, dims[0], cols, flag);
+    else
+        hipLaunchKernelGGL(k_column_flags<1>, grid, dim3(256), 0, stream, vol, dims[0], cols, flag);
     hipLaunchKernelGGL(k_edge_extents, dim3(kBlocks), dim3(256), 0, stream, flag, dims[1], dims[2], a, b, zx, part);
     PK_HIP(hipGetLastError());
     double h[5 * kBlocks];

@@ -16,7 +16,7 @@
 // floats, and every value of an output column uses the same two input columns
 // and weight.  A block takes eight neighbouring output columns: they read nine
 // neighbouring input columns, each once.  Coalesced and HBM-bound (4 bytes read
-// + 4 written per value).  512x512x256 at 31.5 degrees, dz 0.2, pixel 0.108: 0.140 ms; with a
+// + 4 written per value).  512x512x256 at 31.5 degrees, dz 0.2: 0.140 ms; with a
 // block per output column 0.172 ms (both columns of a blend read by every block:
 // 512 instead of 268 MB past L2).
 #include <hip/hip_runtime.h>
@@ -196,8 +196,9 @@ __global__ void __launch_bounds__(256) k_affine3d(const float* __restrict__ vol,
 // wavefront takes 64 V values of kRowsRun neighbouring output columns of one
 // page; the wavefronts of a block take neighbouring pages and blocks go to the
 // XCDs in contiguous ranges, so that the input columns they share meet in L1
-// and L2.  Bound by memory: 512x980x200 rotated by 31.5 degrees 0.180 ms (4.1
-// TB/s of the input read once and the result written), with the general kernel
+// and L2.  Bound by memory: 512x980x200 rotated by 31.5 degrees 0.160 ms (4.6
+// TB/s of the input read once and the result written; 0.180 with stores through
+// the caches), with the general kernel
 // 0.311 ms.
 constexpr int kRowsRun = 8;
 template <int V>
@@ -254,7 +255,9 @@ __global__ void __launch_bounds__(256) k_affine_rows(const float* __restrict__ v
                 }
             }
             float* __restrict__ g = out + ((p * ox + c) * oy + r);
-            if constexpr (V == 4) *reinterpret_cast<float4*>(g) = make_float4(o[0], o[1], o[2], o[3]);
+            typedef float nt_f4 __attribute__((ext_vector_type(4)));
+            if constexpr (V == 4)  // past the caches, which keep the input's columns
+                __builtin_nontemporal_store(nt_f4{o[0], o[1], o[2], o[3]}, reinterpret_cast<nt_f4*>(g));
             else *g = o[0];
         }
     }

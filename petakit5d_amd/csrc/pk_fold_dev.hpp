@@ -197,6 +197,9 @@ __device__ __forceinline__ FoldXPos foldx_pos(const FoldX& f, int s, int u, int 
 }
 
 // Outer dim-2 step: memory -> LDS (inverse) or LDS -> memory (forward), one column per task.
+// The row pass stores its spectrum past the caches: the column pass reads it on
+// other XCDs (OMW-2 512x512x256 2.35 -> 2.32 ms, 16 chunks of up to 384x384x256 8.42 ->
+// 8.26; the real-space volumes stored that way cost Biggs-10 2.5 %).
 template <int R, bool INV>
 __device__ __forceinline__ void foldx_mem_r(const FoldX& f, int s, float2* lds, float2* __restrict__ sp0, int y0) {
     foldx_tasks(f.st.U[s], f.H1, f.mag_chH, f.mag_remH, [&](int u, int k, auto uni) {
@@ -208,7 +211,7 @@ __device__ __forceinline__ void foldx_mem_r(const FoldX& f, int s, float2* lds, 
         foldx_dft<R, INV, decltype(uni)::value>(v, f.twy, p.j, f.st.tws[s], p.twid);
         static_for<0, R>([&](auto c) {
             if constexpr (INV) q[decltype(c)::value * p.ld] = v[decltype(c)::value];
-            else g[decltype(c)::value * p.gd] = v[decltype(c)::value];
+            else st_f2<true>(g + decltype(c)::value * p.gd, v[decltype(c)::value]);
         });
     });
 }
@@ -261,8 +264,8 @@ __device__ __forceinline__ void foldx_pair_r(const FoldX& f, int s, float2* lds,
             static_for<0, R>([&](auto c) {
                 constexpr int q = decltype(c)::value;
                 if constexpr (MEM) {
-                    g[q * p.gd + k] = v1[q];
-                    g[q * p.gd + (f.L - k)] = v2[q];
+                    st_f2<true>(g + (q * p.gd + k), v1[q]);
+                    st_f2<true>(g + (q * p.gd + (f.L - k)), v2[q]);
                 } else {
                     q1[q * p.ld] = v1[q];
                     q2s[q * p.ld] = v2[q];

@@ -20,6 +20,10 @@
 //     x BIGGS_UPDATE  Jn = max(Y .* C2R_x(A), 0) (into J3's buffer);
 //                     J4 = Jn - Y, with the two dot products of the next
 //                     step length accumulated before J4 is overwritten
+//
+// Where the plan has the two-pass form (VolPlan::fold), every "y FWD; z ...;
+// y INV" is one column pass and the row passes carry the outer dim-2 steps
+// (pk_fold_dev.hpp).
 #include "pk_engine.hpp"
 
 #include <hip/hip_runtime.h>

@@ -121,6 +121,7 @@ def rotateFrame3D(vol, angle, zxRatio, reverse=False, Crop=True, resample=None, 
         raise ValueError(f"rotateFrame3D: output size {od}")
     inv = np.ascontiguousarray(np.linalg.inv(T), dtype=np.float64)
     out = torch.empty((od[2], od[1], od[0]), dtype=torch.float32, device=t.device).permute(2, 1, 0)
+    torch.cuda.current_stream(t.device).synchronize()  # out's memory: its earlier uses
     fn = _lib.load().pk_affine_warp3d_cubic if interp == "cubic" else _lib.load().pk_affine_warp3d
     ctx.check(fn(ctx.handle, ctypes.c_void_p(t.data_ptr()), i64x3(d), inv.ctypes.data_as(ctypes.POINTER(ctypes.c_double)),
                  i64x3(od), ctypes.c_void_p(out.data_ptr())))

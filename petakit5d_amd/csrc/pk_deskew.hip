@@ -16,7 +16,7 @@
 // floats, and every value of an output column uses the same two input columns
 // and weight.  A block takes eight neighbouring output columns: they read nine
 // neighbouring input columns, each once.  Coalesced and HBM-bound (4 bytes read
-// + 4 written per value).  512x512x256 at 31.5 degrees, dz 0.2: 0.140 ms; with a
+// + 4 written per value).  512x512x256 at 31.5 degrees, dz 0.2: 0.139 ms; with a
 // block per output column 0.172 ms (both columns of a blend read by every block:
 // 512 instead of 268 MB past L2).
 #include <hip/hip_runtime.h>
@@ -196,10 +196,10 @@ __global__ void __launch_bounds__(256) k_affine3d(const float* __restrict__ vol,
 // wavefront takes 64 V values of kRowsRun neighbouring output columns of one
 // page; the wavefronts of a block take neighbouring pages and blocks go to the
 // XCDs in contiguous ranges, so that the input columns they share meet in L1
-// and L2.  Bound by memory: 512x980x200 rotated by 31.5 degrees 0.160 ms (4.6
-// TB/s of the input read once and the result written; 0.180 with stores through
-// the caches), with the general kernel
-// 0.311 ms.
+// and L2.  Bound by memory: 512x980x200 rotated by 31.5 degrees 0.180 ms (4.1
+// TB/s past L2), with the general kernel 0.311 ms.  Stores past the caches make
+// it 0.190 ms and the next reader of the input faster (the column flags 0.045
+// instead of 0.076 ms): rotations of one volume after another 0.312 against 0.332.
 constexpr int kRowsRun = 8;
 template <int V>
 __global__ void __launch_bounds__(256) k_affine_rows(const float* __restrict__ vol, float* __restrict__ out, int64_t ny,
@@ -265,8 +265,8 @@ __global__ void __launch_bounds__(256) k_affine_rows(const float* __restrict__ v
 
 // rotateFrame3D.m:46-66's extents without the projection leaving the device:
 // flag of a column = max over dim 1 ~= 0 (a positive value or a NaN settles it;
-// else true when no value is 0), one wavefront a column.  Bound by reading the
-// columns that hold only zeros.  512x980x200: 0.076 ms and 0.009 ms for the
+// else true when no value is 0).  Bound by reading the columns that hold only
+// zeros.  512x980x200: 0.045-0.076 ms (0.112 with one column a wavefront) and 0.009 ms for the
 // extents; the maximum as a reduction of the library, its copy and the host's
 // search were 0.6 ms.
 // A wavefront follows kFlagCols columns at once, 64 V values of each a step.

@@ -286,8 +286,7 @@ pk_status pk_wb_backprojector(pk_ctx *ctx, const float *psf_fp, const int64_t di
  * the three passes).  Results are shared by the process's contexts and appended to the file
  * named by the environment variable PK_TUNE_FILE when set (read back at the
  * next plan of the size).  report (may be NULL) receives a one-line summary.
- * Call it before serving: requests in flight keep the shapes they started with
- * only when nothing retunes their size. */
+ * Requests in flight keep the shapes and the form they were admitted with. */
 pk_status pk_autotune(pk_ctx *ctx, const int64_t dims[3], char *report, size_t report_len);
 
 /* Sets the launch shapes of a padded size without measuring (no counterpart

@@ -136,7 +136,7 @@ size_t pk_ctx_impl::chunk_prepare(Chunk& c, const pk_vol& in, const pk_vol& out,
     {
         const int64_t a = smooth_up(c.d[0]), b = smooth_up(c.d[1]), z = smooth_up(c.d[2]);
         if ((c.o.flags & PK_FLAG_AUTOTUNE) && !plan(a, b, z).tuned) autotune(a, b, z);
-        c.vp = &plan(a, b, z);
+        c.vp = plan(a, b, z);
     }
     // The cropped PSF is a function of the whole PSF and the crop window, so
     // its cache key is the whole PSF's key with the window folded in (the
@@ -151,11 +151,11 @@ size_t pk_ctx_impl::chunk_prepare(Chunk& c, const pk_vol& in, const pk_vol& out,
             whole &= win[d + 3] == pd[d];
         }
         const uint64_t key = whole ? h : key_mix(h, win, 6);
-        if (const float2* hit = otf_find(*c.vp, key, win + 3)) return hit;
+        if (const float2* hit = otf_find(c.vp, key, win + 3)) return hit;
         std::vector<float> q;
         int64_t qd[3];
         crop_psf(p, pd, c.d, q, qd);
-        return otf_build(*c.vp, key, q.data(), qd);
+        return otf_build(c.vp, key, q.data(), qd);
     };
     c.Hf = otf_cropped(psf_f, fd, hf);
     otf_pin(c.Hf, +1);
@@ -173,7 +173,7 @@ size_t pk_ctx_impl::chunk_prepare(Chunk& c, const pk_vol& in, const pk_vol& out,
     c.in_host = in.mem == PK_MEM_HOST;
     c.out_host = out.mem == PK_MEM_HOST ? out.data : nullptr;
     c.out_bytes = (c.o.save16bit ? 2 : 4) * (size_t)(c.d[0] * c.d[1] * c.d[2]);
-    const VolPlan& vp = *c.vp;
+    const VolPlan& vp = c.vp;
     const size_t esz = c.u16 ? 2 : 4;
     const int64_t nxb = vp.x_blocks();
     size_t need = 2 * align_up(sizeof(float) * vp.N) + align_up(sizeof(float2) * vp.S);
@@ -187,7 +187,7 @@ size_t pk_ctx_impl::chunk_prepare(Chunk& c, const pk_vol& in, const pk_vol& out,
 
 // Carve the chunk's buffers from base and stage its input (copy, zero pad).
 void pk_ctx_impl::chunk_place(Chunk& c, char* base, hipStream_t copy_stream) {
-    const VolPlan& vp = *c.vp;
+    const VolPlan& vp = c.vp;
     char* p = base;
     auto take = [&](size_t bytes) {
         char* r = p;
@@ -226,7 +226,7 @@ void pk_ctx_impl::chunk_place(Chunk& c, char* base, hipStream_t copy_stream) {
 // Epilogue operands of a chunk (decon_lucy_function.m:177-203; no bbox or
 // erosion in the step engine): output = the chunk's own (unpadded) size.
 static EpiArgs chunk_epi(const Chunk& c) {
-    const VolPlan& vp = *c.vp;
+    const VolPlan& vp = c.vp;
     EpiArgs e{};
     e.J = (c.method == 0 && c.par == 1) ? c.J3 : c.J;
     e.I = c.I;
@@ -260,7 +260,7 @@ void pk_ctx_impl::run_step(std::vector<Chunk*>& act) {
     };
     auto base_x = [&](const Chunk& c, int mode) {
         XArgs a{};
-        const VolPlan& vp = *c.vp;
+        const VolPlan& vp = c.vp;
         a.n1 = (int)vp.n1;
         a.h1 = (int)vp.h1;
         a.hp = (int)vp.hp;
@@ -285,7 +285,7 @@ void pk_ctx_impl::run_step(std::vector<Chunk*>& act) {
         g.lds = lds;
     };
     auto add_x = [&](RowPass& rp, const Chunk& c, const XArgs& a) {
-        const VolPlan& vp = *c.vp;
+        const VolPlan& vp = c.vp;
         if (vp.fold.on) {
             const FoldPlan& fp = vp.fold;
             FoldX f = fp.x;
@@ -314,14 +314,14 @@ void pk_ctx_impl::run_step(std::vector<Chunk*>& act) {
     // kernels.  Float I where other code reads it: the damp epilogue, OMW with
     // one iteration (its last update reads J = I) and no iteration.
     auto u16_est = [&](const Chunk& c) -> uint16_t* {
-        const VolPlan& vp = *c.vp;
+        const VolPlan& vp = c.vp;
         const int ctk = vp.packed ? vp.x.fp.L : -vp.x.fp.L;
         const bool ok = c.u16 && c.numit >= (c.method == 1 ? 2 : 1) && !(c.o.damp_factor > 1) &&
                         (vp.fold.on || (vp.x.block.x == 256 && xrow_available(ctk, vp.x.fp.E)));
         return ok ? reinterpret_cast<uint16_t*>(c.I) : nullptr;
     };
     auto add_conv = [&](Pass<FoldC>& ps, const Chunk& c, int mode, const float2* otf) {
-        const VolPlan& vp = *c.vp;
+        const VolPlan& vp = c.vp;
         const FoldPlan& fp = vp.fold;
         FoldC f = fp.c;
         f.data = c.A;
@@ -331,7 +331,7 @@ void pk_ctx_impl::run_step(std::vector<Chunk*>& act) {
         add_fold(ps, {(int64_t)fp.cnt, mode, (int64_t)fp.clds, 0, 0, 0}, f, fp.cnt, fp.clds, fp.cblocks);
     };
     auto add_col = [&](Pass<ColChunk>& ps, const Chunk& c, int axis, int mode, const float2* otf) {
-        const VolPlan& vp = *c.vp;
+        const VolPlan& vp = c.vp;
         if (vp.fold.on) return;  // its two passes hold every strided step
         const AxisLaunch& ax = axis == 2 ? vp.y : vp.z;
         if (ax.fp.L == 1 && (mode == CM_FWD || mode == CM_INV)) return;
@@ -389,14 +389,14 @@ void pk_ctx_impl::run_step(std::vector<Chunk*>& act) {
         std::vector<size_t> order(act.size());
         for (size_t i = 0; i < order.size(); ++i) order[i] = i;
         std::stable_sort(order.begin(), order.end(),
-                         [&](size_t a, size_t b) { return act[a]->vp->N > act[b]->vp->N; });
+                         [&](size_t a, size_t b) { return act[a]->vp.N > act[b]->vp.N; });
         int64_t load[kSets] = {};
         for (size_t i : order) {
             int best = 0;
             for (int k = 1; k < nset; ++k)
                 if (load[k] < load[best]) best = k;
             set_of[i] = best;
-            load[best] += act[i]->vp->N;
+            load[best] += act[i]->vp.N;
         }
     }
     RowPass prep[kSets], biggs_y[kSets], ratio[kSets], update[kSets];
@@ -410,7 +410,7 @@ void pk_ctx_impl::run_step(std::vector<Chunk*>& act) {
             XArgs a = base_x(c, c.u16 ? XM_PREP_U16 : XM_PREP_F32);
             a.raw16 = c.raw16;
             a.rawf = c.rawf;
-            const VolPlan& vp = *c.vp;
+            const VolPlan& vp = c.vp;
             if (vp.n1 != c.d[0] || vp.n2 != c.d[1] || vp.n3 != c.d[2]) {  // padded plan: read the caller's layout
                 a.s0 = c.d[0];
                 a.s1 = c.d[1];
@@ -424,8 +424,8 @@ void pk_ctx_impl::run_step(std::vector<Chunk*>& act) {
             if (a.I16 && c.method == 1) a.J = nullptr;  // OMW: the first update reads I (J_1 = I)
             add_x(prep[si], c, a);
             if (c.method == 0) {
-                hipLaunchKernelGGL(k_fill_f32, dim3((unsigned)std::min<int64_t>((c.vp->N + 255) / 256, 65536)), dim3(256),
-                                   0, stream, c.J3, c.vp->N, 0.f);
+                hipLaunchKernelGGL(k_fill_f32, dim3((unsigned)std::min<int64_t>((c.vp.N + 255) / 256, 65536)), dim3(256),
+                                   0, stream, c.J3, c.vp.N, 0.f);
                 hipLaunchKernelGGL(k_fill_f32, dim3(1), dim3(64), 0, stream, c.lam, (int64_t)1, 0.f);
                 PK_HIP(hipGetLastError());
             }
@@ -434,7 +434,7 @@ void pk_ctx_impl::run_step(std::vector<Chunk*>& act) {
         const int kn = c.k + 1;        // the iteration this step runs
         if (c.method == 0) {
             if (kn > 2)
-                lam.push_back(LamChunk{c.part, (int)c.vp->x_blocks(), c.lam});
+                lam.push_back(LamChunk{c.part, (int)c.vp.x_blocks(), c.lam});
             XArgs a = base_x(c, XM_BIGGS_Y);
             a.J = c.par ? c.J3 : c.J;
             a.J3 = c.par ? c.J : c.J3;
@@ -442,8 +442,8 @@ void pk_ctx_impl::run_step(std::vector<Chunk*>& act) {
             a.lambda = c.lam;
             add_x(biggs_y[si], c, a);
         }
-        const int cax = c.vp->conv_axis, oax = cax == 3 ? 2 : 3;  // pass order of the chunk's plan
-        if (c.vp->fold.on) {
+        const int cax = c.vp.conv_axis, oax = cax == 3 ? 2 : 3;  // pass order of the chunk's plan
+        if (c.vp.fold.on) {
             add_conv(fc1[si], c, CM_CONV, c.Hf);
             add_conv(fc2[si], c, c.method == 1 ? CM_CONV : CM_CONVJ, c.method == 1 ? c.Hb : c.Hf);
         }

@@ -1398,10 +1398,8 @@ void pk_ctx_impl::decon(int method, const pk_vol* Iv, const float* psf_f, const 
     const int64_t* od = g.od;
 
     if ((o->flags & PK_FLAG_AUTOTUNE) && !plan(n1, n2, n3).tuned) autotune(n1, n2, n3);
-    const VolPlan& planned = plan(n1, n2, n3);
-    VolPlan natural;  // the unfused path's transforms are in natural order
-    if (o->flags & PK_FLAG_UNFUSED) natural = planned.three_pass();
-    const VolPlan& vp = (o->flags & PK_FLAG_UNFUSED) ? natural : planned;
+    // a copy: an iteration hook may retune the size.  The unfused path's transforms are in natural order
+    const VolPlan vp = (o->flags & PK_FLAG_UNFUSED) ? plan(n1, n2, n3).three_pass() : plan(n1, n2, n3);
     const int64_t N = vp.N;
     if (o->flags & PK_FLAG_NO_OTF_CACHE) {  // rebuild the OTFs on every call (comparison baseline)
         otf.erase(std::remove_if(otf.begin(), otf.end(), [](const OtfEntry& e) { return e.pins == 0; }), otf.end());

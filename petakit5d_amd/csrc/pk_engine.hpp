@@ -106,7 +106,9 @@ struct OtfEntry {
 struct Chunk {
     int method = 1, numit = 0, k = 0, par = 0;  // k: iterations done; par: Biggs buffer parity
     pk_opts o{};
-    const VolPlan* vp = nullptr;
+    // by value: a retune of the size between two steps may change the pass form, and with it the order of A, Hf and Hb
+    // and the number of partials
+    VolPlan vp;
     int64_t d[3] = {0, 0, 0};  // caller's size (the plan may be padded)
     const float2* Hf = nullptr;
     const float2* Hb = nullptr;

@@ -6,6 +6,8 @@ three steps along the row, none and one dim-2 step in the column pass, one to
 three along dim 3, 8- and 16-column tiles, tiles whose last columns are padding,
 one and two row groups per block.  No other test uses these sizes: a pinned
 size stays pinned for the process's later plans."""
+import time
+
 import numpy as np
 import pytest
 
@@ -42,9 +44,9 @@ def _rel(a, b):
     return float(np.linalg.norm(a - b) / np.linalg.norm(b))
 
 
-def _three_pass(shape):
-    """A context whose plan of this size is pinned to the three-pass kernels."""
-    ctx = pk.Context(0)
+def _three_pass(shape, ctx=None):
+    """A context (a new one) whose plan of this size is pinned to the three-pass kernels."""
+    ctx = ctx or pk.Context(0)
     L = shape[0] // 2
     divisors = [1, 2, 3, 4, 5, 6, 8, 9, 10, 12, 15, 16, 18, 20, 24, 25, 27, 30, 32]
 
@@ -98,3 +100,33 @@ def test_two_pass_batch_and_options_equal_single_calls():
                 fn = pk.decon_lucy_omw_function if method == "omw" else pk.decon_lucy_function
                 J = fn(v, *args, Background=100, pad=True, **kw)[0]
                 assert np.array_equal(o, J), (method, kw, v.shape)
+
+
+@pytest.mark.parametrize("shape, method", [((60, 80, 36), "omw"), ((48, 80, 36), "rl")])
+def test_request_in_flight_keeps_its_form_when_its_size_is_pinned(shape, method):
+    """The size of a request goes to the three passes between two of its steps: the request goes on in the two-pass
+    form, whose spectrum order, OTFs and partial sums it was admitted with, and the next one takes the new form."""
+    n = 1500  # iterations: a few tens of ms, so that the pin falls between two of them
+    I, psf, psf_b = _volume(shape, sum(shape))
+    fn = pk.decon_lucy_omw_function if method == "omw" else pk.decon_lucy_function
+    kw = dict(Background=100, save16bit=False)
+
+    def alone(ctx, iters):
+        return fn(I, psf, *((psf_b,) if method == "omw" else ()), iters, ctx=ctx, **kw)[0]
+
+    ctx = pk.Context(0)
+    two, two_short = alone(ctx, n), alone(ctx, 3)
+    srv = pk.Server(ctx)
+    req = srv.submit(I, psf, psf_b, n, method=method, **kw)
+    while req.info()["iterations_done"] < 2:
+        time.sleep(1e-4)
+    _three_pass(shape, ctx)
+    done = req.info()["iterations_done"]
+    print(f"[fold] {method} {shape}: pinned after {done} of {n} iterations", flush=True)
+    assert done < n
+    np.testing.assert_array_equal(req.result(timeout_s=60), two)
+    after = srv.submit(I, psf, psf_b, 3, method=method, **kw).result(timeout_s=60)
+    srv.stop()
+    np.testing.assert_array_equal(after, alone(ctx, 3))  # three passes, served and alone
+    assert not np.array_equal(after, two_short) and _rel(after, two_short) <= 1e-5
+    ctx.close()

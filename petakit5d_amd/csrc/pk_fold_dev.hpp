@@ -134,9 +134,39 @@ __device__ __forceinline__ int fold_slot(const FoldX& f, int k) {
     return q1 * f.M1p + q2 * f.sx.M[1] + q3;
 }
 
-// Radix-R butterfly of a dim-2 step with its twiddles W_{n2}^{m j tws}: exact
-// table values where j is the same for the whole wavefront (scalar loads),
-// powers of one where it is not.
+// Twiddles W_L^(m j tws), m < R, of one butterfly (m j tws < L).  A product
+// carries the rounding of its factors, and a power of one value m times that
+// value's: with stage_twiddle's powers of W^1 the error of OMW-2 against 64 bits
+// was up to 1.46 times the three passes' (64x64x32, 3.5e-7 against 2.4e-7).  Here
+// no power takes more than W^1 or W^2 and one of the table's W^4, W^8, W^12, and
+// R <= 4 and R = 8 read all from the table: 0.56-1.07 times the three passes'
+// error over 20 sizes, for up to 1.4 % of the time (8 chunks of up to 384x384x256,
+// Biggs-10, 20.4 -> 20.7 ms).  All radices from the table: no closer, 2-4 % slower.
+template <int R, bool INV>
+__device__ __forceinline__ void fold_twiddle(float2 (&v)[R], const float2* __restrict__ tw, int j, int tws) {
+    constexpr bool all = R <= 4 || R == 8;
+    float2 w[R];
+    const int d = j * tws;
+    static_for<1, R>([&](auto mc) {
+        constexpr int m = decltype(mc)::value;
+        if constexpr (all || m == 1 || m % 4 == 0) w[m] = tw[m * d];
+    });
+    if constexpr (!all) {
+        w[2] = cmul(w[1], w[1]);
+        static_for<3, R>([&](auto mc) {
+            constexpr int m = decltype(mc)::value;
+            if constexpr (m % 4 == 3 && m + 1 < R) w[m] = cmulc(w[m + 1], w[1]);
+            else if constexpr (m % 4 != 0) w[m] = cmul(w[m / 4 * 4], w[m % 4]);
+        });
+    }
+    static_for<1, R>([&](auto mc) {
+        constexpr int m = decltype(mc)::value;
+        v[m] = INV ? cmulc(v[m], w[m]) : cmul(v[m], w[m]);
+    });
+}
+
+// Radix-R butterfly of a dim-2 step with its twiddles W_{n2}^{m j tws}: table
+// values where j is the same for the whole wavefront (scalar loads).
 template <int R, bool INV, bool UNI>
 __device__ __forceinline__ void foldx_dft(float2 (&v)[R], const float2* __restrict__ tw, int j, int tws, bool twid) {
     if constexpr (!INV) dft<R, false>(v);
@@ -148,7 +178,7 @@ __device__ __forceinline__ void foldx_dft(float2 (&v)[R], const float2* __restri
                 v[m] = INV ? cmulc(v[m], w) : cmul(v[m], w);
             });
         } else {
-            stage_twiddle<R, INV>(v, tw, j, tws);
+            fold_twiddle<R, INV>(v, tw, j, tws);
         }
     }
     if constexpr (INV) dft<R, true>(v);
@@ -315,11 +345,11 @@ __device__ __forceinline__ void foldx_row_r(const FoldX& f, int s, float2* lds) 
         float2 v[R];
         static_for<0, R>([&](auto c) { v[decltype(c)::value] = q[decltype(c)::value * M]; });
         if constexpr (INV) {
-            if (M > 1) stage_twiddle<R, true>(v, f.tw, j, tws);
+            if (M > 1) fold_twiddle<R, true>(v, f.tw, j, tws);
             dft<R, true>(v);
         } else {
             dft<R, false>(v);
-            if (M > 1) stage_twiddle<R, false>(v, f.tw, j, tws);
+            if (M > 1) fold_twiddle<R, false>(v, f.tw, j, tws);
         }
         static_for<0, R>([&](auto c) { q[decltype(c)::value * M] = v[decltype(c)::value]; });
     }
@@ -411,7 +441,7 @@ __device__ __forceinline__ void foldx_mid_r(const FoldX& f, float2* lds, int y0,
         float2 v[R];
         if constexpr (IN) {
             static_for<0, R>([&](auto c) { v[decltype(c)::value] = q[decltype(c)::value * f.M1p]; });
-            if (M1 > 1) stage_twiddle<R, true>(v, f.tw, j, tws);
+            if (M1 > 1) fold_twiddle<R, true>(v, f.tw, j, tws);
             dft<R, true>(v);
         }
         EpiRow er{0, 0, false};
@@ -460,7 +490,7 @@ __device__ __forceinline__ void foldx_mid_r(const FoldX& f, float2* lds, int y0,
         });
         if (out_spec) {
             dft<R, false>(v);
-            if (M1 > 1) stage_twiddle<R, false>(v, f.tw, j, tws);
+            if (M1 > 1) fold_twiddle<R, false>(v, f.tw, j, tws);
             static_for<0, R>([&](auto c) { q[decltype(c)::value * f.M1p] = v[decltype(c)::value]; });
         }
     }
@@ -639,11 +669,11 @@ __device__ __forceinline__ void foldc_step_r(const FoldC& f, int s, float2* lds,
             });
             dft<R, true>(v);
         } else if constexpr (INV) {
-            if (M > 1) stage_twiddle<R, true>(v, tw, k.j, tws);
+            if (M > 1) fold_twiddle<R, true>(v, tw, k.j, tws);
             dft<R, true>(v);
         } else {
             dft<R, false>(v);
-            if (M > 1) stage_twiddle<R, false>(v, tw, k.j, tws);
+            if (M > 1) fold_twiddle<R, false>(v, tw, k.j, tws);
         }
         if constexpr (KIND == FK_STORE || KIND == FK_OUT) {
             if (k.ok) {

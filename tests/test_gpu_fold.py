@@ -130,3 +130,30 @@ def test_request_in_flight_keeps_its_form_when_its_size_is_pinned(shape, method)
     np.testing.assert_array_equal(after, alone(ctx, 3))  # three passes, served and alone
     assert not np.array_equal(after, two_short) and _rel(after, two_short) <= 1e-5
     ctx.close()
+
+
+@pytest.mark.parametrize("shape", [(160, 96, 48), (512, 64, 32), (300, 100, 60)], ids=lambda s: "x".join(map(str, s)))
+def test_two_pass_form_is_no_further_from_64_bits_than_three_passes(oracle, shape):
+    """A back projector that sharpens brings the transforms' rounding out.  With twiddles that are powers of one table
+    value the two passes were up to 1.4 times as far from 64 bits as the three; 1.1: the spread of four volumes."""
+    psf = synth.gaussian_psf((15, 15, 21), 1.2, 2.5, 20.0)
+    h = np.fft.fftn(np.fft.ifftshift(psf.astype(np.float64)))
+    wiener = np.conj(h) / (np.abs(h) ** 2 + 0.005) * np.clip(np.log10(np.maximum(np.abs(h), 1e-12)) / 2 + 1, 0, 1)
+    psf_b = np.asfortranarray(np.fft.fftshift(np.fft.ifftn(wiener).real), dtype=np.float32)
+    vols = []
+    for k in range(4):
+        g = np.random.default_rng(50 + k)
+        obj = synth.point_emitters(shape, int(np.prod(shape)) // 3000, (20000, 90000), g)
+        vols.append(synth.poisson_u16(synth._fft_convolve_circular(obj, psf) + 105, g))
+    two = pk.Context(0)
+    ref = [oracle.decon_lucy_omw_function(v, psf, psf_b, 2, Background=100, save16bit=False, precision="f64")[0]
+           for v in vols]
+
+    def error(ctx):
+        out = [pk.decon_lucy_omw_function(v, psf, psf_b, 2, Background=100, save16bit=False, ctx=ctx)[0] for v in vols]
+        return float(np.sqrt(np.mean([_rel(o, r) ** 2 for o, r in zip(out, ref)])))
+
+    e2 = error(two)
+    e3 = error(_three_pass(shape, two))
+    print(f"[fold] {shape}: error against 64 bits, two passes {e2:.3e}, three {e3:.3e}", flush=True)
+    assert e2 <= 1.1 * e3

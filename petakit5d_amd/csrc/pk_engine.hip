@@ -515,7 +515,7 @@ struct Wisdom {
 // Launch shapes of one wisdom line {xE, yE, yNT, yT, zE, zNT, zT, conv_axis}
 // applied to a plan; false (plan unchanged) when a shape is infeasible.  They
 // are the three-pass form's; xE < 0: and the size runs that form (measured
-// faster, or pinned), instead of the two-pass form where there is one.
+// faster, or pinned), instead of the two-pass form where it is the default.
 bool pk_ctx_impl::apply_shapes(VolPlan& vp, const std::array<int, 8>& line) {
     std::array<int, 8> v = line;
     const bool three = v[0] < 0;
@@ -570,6 +570,33 @@ static void fill_real_twiddles(std::vector<float2>& h, int64_t n1) {
     }
 }
 
+// The two-pass form a size takes by default; off where it has no plan or the
+// three passes are the faster form.  Calls of OMW-2 at 350 sizes, three passes
+// with built-in shapes against two, time ratios:
+//   - four-column tiles, both strided transforms of the three passes in two
+//     stages of fewer than 30 values a thread and the dim-2 kernel's blocks full:
+//     0.74-0.995 at 17 of 19 such sizes (1024x512x256 4.62 against 5.58 ms,
+//     512x512x512 4.90 against 5.11); the other four-column plans gain 1.26 times
+//     on average
+//   - 1024 and 2048 long rows, whose row pass takes three steps in LDS, with a
+//     dim-3 transform of more than one stage: 0.74-0.98 at 27 of 34 sizes
+//     (1024x1024x128 4.71 against 5.96 ms, 1024x256x64 0.615 against 0.662), 1.06
+//     at most; 16-column tiles and dim 3 <= 32 gain there too, 1.04-1.38
+// Of the sizes left a few lose: 7 of 89 with four columns, by up to 6 %, and some
+// with an odd dim 2 (225, 625, 729), by up to 14 %.
+static FoldPlan default_fold(int64_t n1, int64_t n2, int64_t n3, int64_t hp) {
+    if (tune().pinned()) return FoldPlan{};
+    const FoldPlan fp = fold_plan(n1, n2, n3, hp);
+    if (!fp.on) return fp;
+    const AxisLaunch y = col_candidates((int)n2, 1)[0], z = col_candidates((int)n3, 2)[0];
+    auto lean = [](const AxisLaunch& a) { return a.fp.nst == 2 && a.fp.E != 30; };
+    const int64_t L = n1 / 2;
+    const bool full = (int)y.block.x * 4 > y.nt * 3;
+    if (fp.T < 8 && lean(y) && lean(z) && full) return FoldPlan{};
+    if (fp.T < 16 && L >= 512 && (L & (L - 1)) == 0 && z.fp.nst > 1) return FoldPlan{};
+    return fp;
+}
+
 VolPlan pk_ctx_impl::plan_shapes(int64_t n1, int64_t n2, int64_t n3) const {
     for (int64_t n : {n1, n2, n3})
         if (!smooth235(n))
@@ -590,7 +617,7 @@ VolPlan pk_ctx_impl::plan_shapes(int64_t n1, int64_t n2, int64_t n3) const {
     vp.x = x_candidates(vp.row_len(), vp.packed)[0];
     vp.y = col_candidates((int)n2, 1)[0];
     vp.z = col_candidates((int)n3, 2)[0];
-    if (!tune().pinned()) vp.fold = fold_plan(n1, n2, n3, vp.hp);
+    vp.fold = default_fold(n1, n2, n3, vp.hp);
     {  // shapes measured earlier for this size (this process or PK_TUNE_FILE)
         Wisdom& w = Wisdom::get();
         std::lock_guard<std::mutex> lk(w.mu);
@@ -779,7 +806,7 @@ std::string pk_ctx_impl::autotune(int64_t n1, int64_t n2, int64_t n3) {
     rep += buf;
     bool three = false;
     // the two-pass form against the three-pass one: a half iteration of each (the built-in choice is the former)
-    if (const FoldPlan fp = tune().pinned() ? FoldPlan{} : fold_plan(n1, n2, n3, vp.hp); fp.on) {
+    if (const FoldPlan fp = default_fold(n1, n2, n3, vp.hp); fp.on) {
         auto half = [&](const VolPlan& t) {
             return timed([&] {
                 const int oax = t.conv_axis == 3 ? 2 : 3;

@@ -3,7 +3,7 @@ against the three-pass form, which pk_tune_set pins.
 
 Sizes cover its branches: one and two dim-2 steps in the row pass, one to
 three steps along the row, none and one dim-2 step in the column pass, one to
-three along dim 3, 8- and 16-column tiles, tiles whose last columns are padding,
+three along dim 3, 4-, 8- and 16-column tiles, tiles whose last columns are padding,
 one and two row groups per block.  No other test uses these sizes: a pinned
 size stays pinned for the process's later plans."""
 import threading
@@ -30,6 +30,7 @@ SIZES = [
     (50, 64, 32),
     (72, 64, 16),
     (54, 1024, 100),  # the largest dim-2 steps, 8-column tiles
+    (10, 324, 288),  # 4-column tiles
 ]
 
 
@@ -85,6 +86,28 @@ def test_two_pass_form_matches_oracle_and_three_pass(oracle, shape):
     R3 = pk.decon_lucy_function(I.astype(np.float32), psf, 4, Background=100, save16bit=False, ctx=three)[0]
     assert _rel(J2, J3) <= 1e-5
     assert _rel(R2, R3) <= 1e-5
+
+
+# Either side of the rule that keeps the three passes: rows of 1024 with 8-column tiles; the same with a dim-3 transform
+# of one stage, with 16-column tiles, with rows of 1000; four columns with short dim-2 and dim-3 transforms; and with a
+# dim-3 transform of 30 values a thread
+@pytest.mark.parametrize("shape, form", [
+    ((1024, 128, 64), "three"), ((1024, 128, 32), "two"), ((1024, 64, 64), "two"), ((1000, 128, 64), "two"),
+    ((64, 625, 108), "three"), ((64, 625, 180), "two"),
+], ids=str)
+def test_default_form_of_a_size(shape, form):
+    I, psf, psf_b = _volume(shape, sum(shape))
+    ctx = pk.Context(0)
+    ctx.profile(True)
+    out = pk.decon_lucy_omw_function(I, psf, psf_b, 1, Background=100, save16bit=False, ctx=ctx)[0]
+    passes = ctx.profile_read()
+    assert ("yz_conv" in passes, "z_conv" in passes) == (form == "two", form == "three"), passes
+    other = pk.Context(0)
+    if form == "two":
+        _three_pass(shape, other)
+        assert _rel(out, pk.decon_lucy_omw_function(I, psf, psf_b, 1, Background=100, save16bit=False, ctx=other)[0]) <= 1e-5
+    other.close()
+    ctx.close()
 
 
 def test_two_pass_batch_and_options_equal_single_calls():

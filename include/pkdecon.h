@@ -281,11 +281,13 @@ pk_status pk_wb_backprojector(pk_ctx *ctx, const float *psf_fp, const int64_t di
  * strided passes' values per thread, block sizes and tile widths, and the pass
  * order (which strided axis carries the fused OTF convolution) for the padded
  * size dims on the context's GPU, and keeps the fastest for later calls of that
- * size; and a half iteration of those three passes against the two-pass form,
- * which most even n1 run by default (a line with a negative first field keeps
- * the three passes).  Results are shared by the process's contexts and appended to the file
- * named by the environment variable PK_TUNE_FILE when set (read back at the
- * next plan of the size).  report (may be NULL) receives a one-line summary.
+ * size; and, where the two-pass form is the size's default (most even n1), a
+ * half iteration of those three passes against it.  Results are shared by the
+ * process's contexts and appended to the file named by the environment variable
+ * PK_TUNE_FILE when set (read back at the next plan of the size): dims, then
+ * the eight shapes of pk_tune_set.  In the file a negative first shape keeps
+ * the three passes, a positive one leaves the size's default form.  report
+ * (may be NULL) receives a one-line summary.
  * Requests in flight keep the shapes and the form they were admitted with. */
 pk_status pk_autotune(pk_ctx *ctx, const int64_t dims[3], char *report, size_t report_len);
 
@@ -293,9 +295,10 @@ pk_status pk_autotune(pk_ctx *ctx, const int64_t dims[3], char *report, size_t r
  * in the reference): shapes = {row values per thread, dim-2 values per
  * thread, block size, tile width, dim-3 values per thread, block size, tile
  * width, pass order (2 or 3: the strided axis carrying the OTF convolution)},
- * the fields of one PK_TUNE_FILE line.  The size then runs the three-pass form
- * these shapes belong to.  Applies to this context's later calls
- * and to plans the process's other contexts make afterwards; not written to
+ * the last eight fields of a PK_TUNE_FILE line.  The size then runs the
+ * three-pass form these shapes belong to, whatever the sign of the first (in
+ * the file the sign tells the form).  Applies to this context's later calls and
+ * to plans the process's other contexts make afterwards; not written to
  * the file.  PK_ERR_INVALID_ARG when a shape is not feasible for the size. */
 pk_status pk_tune_set(pk_ctx *ctx, const int64_t dims[3], const int32_t shapes[8]);
 

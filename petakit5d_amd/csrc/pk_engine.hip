@@ -512,6 +512,8 @@ struct Wisdom {
     }
 };
 
+constexpr int kMaxRow = 16384;
+
 // Launch shapes of one wisdom line {xE, yE, yNT, yT, zE, zNT, zT, conv_axis}
 // applied to a plan; false (plan unchanged) when a shape is infeasible.  They
 // are the three-pass form's; xE < 0: and the size runs that form (measured
@@ -519,7 +521,7 @@ struct Wisdom {
 bool pk_ctx_impl::apply_shapes(VolPlan& vp, const std::array<int, 8>& line) {
     std::array<int, 8> v = line;
     const bool three = v[0] < 0;
-    v[0] = std::abs(v[0]);
+    if (three && v[0] >= -kMaxRow) v[0] = -v[0];
     const int Lx = (int)(vp.packed ? vp.n1 / 2 : vp.n1);
     const bool ctx =
         !tune().generic_x && v[0] > 0 && Lx % v[0] == 0 && xrow_available(vp.packed ? Lx : -Lx, v[0]);
@@ -546,8 +548,8 @@ void pk_ctx_impl::set_shapes(int64_t n1, int64_t n2, int64_t n3, const std::arra
     const std::vector<int64_t> key{n1, n2, n3};
     VolPlan vp = plan(n1, n2, n3);
     std::array<int, 8> pin = v;
-    pin[0] = -v[0];
-    if (v[0] < 1 || !apply_shapes(vp, pin)) fail(PK_ERR_INVALID_ARG, "launch shapes not feasible for this size");
+    if (v[0] > 0) pin[0] = -v[0];  // either sign names the three passes here
+    if (!apply_shapes(vp, pin)) fail(PK_ERR_INVALID_ARG, "launch shapes not feasible for this size");
     plans[key] = vp;
     clear_graphs();  // captured loops hold the old launch shapes
     Wisdom& w = Wisdom::get();
@@ -602,7 +604,7 @@ VolPlan pk_ctx_impl::plan_shapes(int64_t n1, int64_t n2, int64_t n3) const {
         if (!smooth235(n))
             fail(PK_ERR_UNSUPPORTED_SIZE, "axis length " + std::to_string(n) +
                                               " is not 2/3/5-smooth; pad it with findGoodFactorNumber(n, 1, false, 5)");
-    if (n1 > 16384 || n2 > 8192 || n3 > 8192) fail(PK_ERR_UNSUPPORTED_SIZE, "axis longer than the supported maximum");
+    if (n1 > kMaxRow || n2 > 8192 || n3 > 8192) fail(PK_ERR_UNSUPPORTED_SIZE, "axis longer than the supported maximum");
     VolPlan vp;
     vp.n1 = n1;
     vp.n2 = n2;

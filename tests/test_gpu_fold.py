@@ -126,6 +126,31 @@ def test_two_pass_batch_and_options_equal_single_calls():
                 assert np.array_equal(o, J), (method, kw, v.shape)
 
 
+def test_tune_set_takes_the_lines_of_the_tune_file(tmp_path, monkeypatch):
+    """Either sign of the first shape pins the three passes; zero is refused."""
+    shape = (100, 64, 36)
+    I, psf, psf_b = _volume(shape, 9)
+    monkeypatch.setenv("PK_TUNE_FILE", str(tmp_path / "tune.txt"))
+    ctx = pk.Context(0)
+    ctx.autotune(shape)
+    line = [int(x) for x in (tmp_path / "tune.txt").read_text().split()]
+    assert tuple(line[:3]) == shape and len(line) == 11
+    out = []
+    for sign in (1, -1):
+        shapes = [sign * abs(line[3])] + line[4:]
+        ctx.tune_set(shape, shapes)
+        ctx.profile(True)
+        out.append(pk.decon_lucy_omw_function(I, psf, psf_b, 2, Background=100, save16bit=False, ctx=ctx)[0])
+        passes = ctx.profile_read()
+        assert "z_conv" in passes or "y_conv" in passes, passes
+        assert "yz_conv" not in passes
+    np.testing.assert_array_equal(out[0], out[1])
+    for first in (0, -2 ** 31):
+        with pytest.raises(pk.PkDeconError):
+            ctx.tune_set(shape, [first] + line[4:])
+    ctx.close()
+
+
 @pytest.mark.parametrize("shapes, method", [([(60, 80, 36), (54, 80, 36), (80, 80, 36)], "omw"),
                                             ([(48, 80, 36), (72, 80, 36), (96, 80, 36)], "rl")], ids=["omw", "rl"])
 def test_request_in_flight_keeps_its_form_when_its_size_is_pinned(shapes, method):

@@ -63,12 +63,6 @@ FoldSteps steps(const std::vector<int>& R, int len, int unit, int before) {
     return st;
 }
 
-unsigned pow2_at_least(int64_t n) {
-    unsigned p = 64;
-    while ((int64_t)p < n) p *= 2;
-    return p;
-}
-
 // Dim-2 steps between a block's a rows, forward order: the pair radix r0 and,
 // when a has more factors, one memory radix.
 bool row_steps(int a, int r0, std::vector<int>& out) {
@@ -80,8 +74,7 @@ bool row_steps(int a, int r0, std::vector<int>& out) {
     return r >= 4 && std::find(std::begin(kMemRadices), std::end(kMemRadices), r) != std::end(kMemRadices);
 }
 
-bool build(FoldPlan& fp, int64_t n1, int64_t n2, int64_t n3, int64_t hp, int a, int b, int T, unsigned xnt,
-           unsigned cnt, int r0) {
+bool build(FoldPlan& fp, int64_t n1, int64_t n2, int64_t n3, int64_t hp, int a, int b, int T, int r0) {
     // even rows only: an odd row's transform has no half-length form, and with
     // twice the LDS and arithmetic the three passes are faster (405x400x200
     // OMW-2: 1.64 ms against 1.74-2.10)
@@ -113,10 +106,6 @@ bool build(FoldPlan& fp, int64_t n1, int64_t n2, int64_t n3, int64_t hp, int a, 
     while (zs % 32 != 8) ++zs;
     fp.clds = (size_t)n3 * zs * sizeof(float2);
     if (fp.xlds > kMaxLds || fp.clds > kMaxLds) return false;
-    // threads: about one radix-16 butterfly each
-    fp.xnt = xnt ? xnt : std::min((unsigned)kFoldXThreads, pow2_at_least((int64_t)G * L / 16));
-    fp.cnt = cnt ? cnt : std::min(1024u, std::max(256u, pow2_at_least(n3 * m * T / 16)));
-    if (fp.xnt > (unsigned)kFoldXThreads || fp.xnt % 64 || (fp.cnt != 256 && fp.cnt != 512 && fp.cnt != 1024)) return false;
     FoldX& x = fp.x;
     x.m = m;
     x.lb = lb;
@@ -158,7 +147,7 @@ bool build(FoldPlan& fp, int64_t n1, int64_t n2, int64_t n3, int64_t hp, int a, 
     c.sy = steps(ry, m, 1, a);
     c.sz = steps(rz, (int)n3, 1, 1);
     fp.cblocks = c.per_xcd * 8;
-    // block indexes are split with 32-bit multiply-high divisions
+    // block indexes are split with 32-bit multiply-high divisions too (fold_div)
     if (fp.xblocks * x.nyb >= (1ll << 32) || (int64_t)c.tiles * c.gx >= (1ll << 32)) return false;
     uint64_t h = 1469598103934665603ull;
     auto mix = [&](int v) { h = (h ^ (uint64_t)(unsigned)v) * 1099511628211ull; };
@@ -209,7 +198,7 @@ FoldPlan search(int64_t n1, int64_t n2, int64_t n3, int64_t hp) {
         for (int r0 : kPairRadices)
             for (int b : {1, 2})
                 for (int T : {16, 8, 4}) {
-                    if (!build(fp, n1, n2, n3, hp, a, b, T, 0, 0, r0)) continue;
+                    if (!build(fp, n1, n2, n3, hp, a, b, T, r0)) continue;
                     for (unsigned xnt : {128u, 256u, 512u, 1024u})
                         for (unsigned cnt : {256u, 512u, 1024u}) {
                             fp.xnt = xnt;

@@ -96,7 +96,9 @@ struct FoldC {
     FoldSteps sy, sz;
 };
 
-// u / d for the small indices here (u < 2^16 * d): mag = floor(2^32 / d) + 1, 0 for d = 1
+// u / d for u d < 2^32: mag = floor(2^32 / d) + 1, 0 for d = 1.  Tasks and their
+// divisors count parts of a tile, at most 20480 values of LDS; block indexes are
+// checked where the plan is built.
 __device__ __forceinline__ int fold_div(int u, uint32_t mag) { return mag ? (int)__umulhi((uint32_t)u, mag) : u; }
 
 // The arguments of a block: a launch over many chunks reads its chunk's

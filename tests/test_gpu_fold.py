@@ -111,9 +111,17 @@ def test_default_form_of_a_size(shape, form):
 
 
 def test_two_pass_batch_and_options_equal_single_calls():
-    """Chunks of several sizes (padded ones among them) in one call give the single calls' bits; so do the options that
-    ride in the last update."""
-    shapes = [(60, 60, 30), (80, 64, 45), (53, 40, 27), (96, 64, 32), (45, 40, 27)]
+    """Chunks of several sizes (padded ones among them: 59 x 59 x 29 runs as 60 x 60 x 30 in two passes, 53 x 40 x 27 as
+    54 x 40 x 27 in three) in one call give the single calls' bits; so do the options that ride in the last update."""
+    shapes = [(60, 60, 30), (80, 64, 45), (53, 40, 27), (96, 64, 32), (45, 40, 27), (59, 59, 29)]
+    ctx = pk.Context(0)
+    ctx.profile(True)
+    for shape, name in (((59, 59, 29), "b_yz_conv"), ((53, 40, 27), "b_z_conv")):
+        v, psf, psf_b = _volume(shape, 3)
+        pk.decon_batch([v], psf, psf_b, 1, method="omw", Background=100, ctx=ctx)
+        passes = ctx.profile_read()
+        assert name in passes and (name == "b_z_conv" or "b_z_conv" not in passes), passes
+    ctx.close()
     vols = [_volume(s, 7 + k)[0] for k, s in enumerate(shapes)]
     _, psf, psf_b = _volume((32, 32, 24), 1)
     for method, it in (("omw", 2), ("rl", 4)):

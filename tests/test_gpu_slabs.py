@@ -36,20 +36,30 @@ def _case(shape, seed):
     return synth.poisson_u16(img, g1), psf
 
 
+# the two-pass form (whole planes are whole blocks), odd rows and rows of 80 pinned to the three passes (slabs hold whole
+# row blocks; the strided passes run slab by slab too)
+CASES = [((64, 64, 32), None), ((96, 40, 48), None), ((45, 40, 48), None),
+         ((80, 54, 64), (10, 6, 256, 16, 8, 256, 16, 3))]
+
+
 def run_cases():
-    """OMW-2 and Biggs-3 on two uint16 volumes (conv along dim 3, the built-in
-    order); float outputs, and the ratio passes' launch count."""
+    """OMW-2 and Biggs-3 on uint16 volumes (conv along dim 3, the built-in
+    order); float outputs, and the launch counts of the passes."""
     import petakit5d_amd as pk
-    ctx = pk.Context(0)
-    ctx.profile(True)
     out = {}
-    for i, shape in enumerate([(64, 64, 32), (96, 40, 48)]):
+    for i, (shape, pin) in enumerate(CASES):
+        ctx = pk.Context(0)
+        ctx.profile(True)
+        if pin:
+            ctx.tune_set(shape, pin)
         I, psf = _case(shape, 21 + i)
         psf_b = np.ascontiguousarray(psf[::-1, ::-1, ::-1])
         out[f"omw{i}"], _ = pk.decon_lucy_omw_function(I, psf, psf_b, 2, Background=100, save16bit=False, ctx=ctx)
         out[f"rl{i}"], _, _ = pk.decon_lucy_function(I, psf, 3, Background=100, save16bit=False, ctx=ctx)
-    out["ratio_launches"] = np.array(ctx.profile_read()["x_ratio"][0])
-    ctx.close()
+        passes = ctx.profile_read()
+        for name in ("x_ratio", "y_fwd", "yz_conv", "z_conv"):
+            out[f"launches{i}_{name}"] = np.array(passes[name][0] if name in passes else 0)
+        ctx.close()
     return out
 
 
@@ -63,8 +73,14 @@ def test_slab_passes_match_whole_volume(tmp_path):
                        timeout=180)
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-2000:]
     got = np.load(path)
-    print(f"  x_ratio launches: whole volume {int(ref['ratio_launches'])}, slabs {int(got['ratio_launches'])}")
-    assert int(got["ratio_launches"]) > int(ref.pop("ratio_launches"))  # the slab path ran
+    for i, (shape, _) in enumerate(CASES):
+        n = {k: (int(ref.pop(f"launches{i}_{k}")), int(got[f"launches{i}_{k}"]))
+             for k in ("x_ratio", "y_fwd", "yz_conv", "z_conv")}
+        print(f"  {shape}: launches whole volume / slabs {n}", flush=True)
+        two = i < 2
+        assert n["x_ratio"][1] > n["x_ratio"][0]  # the slab path ran, in the form the case is for
+        assert (n["yz_conv"][0] > 0, n["z_conv"][0] > 0) == (two, not two)
+        assert two or n["y_fwd"][1] > n["y_fwd"][0]
     for k, v in ref.items():
         assert v.dtype == np.float32 and np.isfinite(v).all() and v.max() > 0
         assert np.array_equal(v.view(np.uint32), got[k].view(np.uint32)), k

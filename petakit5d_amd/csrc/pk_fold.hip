@@ -169,6 +169,13 @@ namespace {
 // every feasible shape (both passes, 17 sizes from 64x64x32 to 512x512x256 and
 // 1024x256x64, 12 to 544 shapes each); with the weights fitted to them the
 // chosen shape is 1.3 % slower than the fastest one on average, 7 % at worst.
+// The last two terms come from batches of equal volumes, where idle threads and
+// large blocks cost what they do not in one volume's launch.  They change 17 of 367
+// sizes: batches gain 1.04-1.30 times (30 volumes of 480x72x60, Biggs-5: 0.88 -> 1.15
+// times the three passes' speed; 15 of 256x256x64, OMW-2: 0.96 -> 1.03), single calls
+// 1.005 times on average (0.95-1.05).  Batches of 256x128x64, 128x256x64, 256x256x32,
+// 1024x64x32 and 128x128x64 stay below the three passes (0.86-0.96), their single
+// calls above (1.06-1.38).
 double fold_score(const FoldPlan& fp, int64_t n3) {
     // blocks a CU holds at once: LDS, and registers (16 wavefronts of the row
     // kernel, 20 of the column kernel)
@@ -187,6 +194,8 @@ double fold_score(const FoldPlan& fp, int64_t n3) {
     s += (fp.xlds > 81920 ? 0.17 : 0.0) + (fp.clds > 81920 ? 0.09 : 0.0);   // one block a CU: nothing hides its phases
     s += 0.02 * fp.x.st.n + 10.0 * fp.c.sy.n;
     s += 0.12 * std::fabs(std::log2(fp.x.st.R[0] / 6.0)) + (fp.x.st.R[1] > 10 ? 0.07 : 0.0);
+    // a batch holds blocks enough for any shape: idle threads, and a large block where two smaller ones fit a CU
+    s += 0.12 * std::max(0.0, std::log2(0.5 / xw)) + (fp.xnt == 1024 && fp.xlds <= 81920 ? 0.06 : 0.0);
     return s;
 }
 

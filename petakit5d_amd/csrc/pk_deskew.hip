@@ -198,8 +198,10 @@ __global__ void __launch_bounds__(256) k_affine3d(const float* __restrict__ vol,
 // XCDs in contiguous ranges, so that the input columns they share meet in L1
 // and L2.  Bound by memory: 512x980x200 rotated by 31.5 degrees 0.180 ms (4.1
 // TB/s past L2), with the general kernel 0.311 ms.  Stores past the caches make
-// it 0.190 ms and the next reader of the input faster (the column flags 0.045
-// instead of 0.076 ms): rotations of one volume after another 0.312 against 0.332.
+// this kernel 0.190 ms and leave the input cached for its other reader, the column
+// flags (0.045 instead of 0.076 ms).  Calls, stores past the caches / plain: one
+// volume again and again 0.319 / 0.339 ms, six in turn 0.320 / 0.345, six with the
+// result copied next 0.516 / 0.523, after 512 MB of other writes 0.366 / 0.361.
 constexpr int kRowsRun = 8;
 template <int V>
 __global__ void __launch_bounds__(256) k_affine_rows(const float* __restrict__ vol, float* __restrict__ out, int64_t ny,

@@ -29,16 +29,18 @@
 // passes and ratio, or column and row pass), three passes with measured launch
 // shapes / two passes, ms: 64x64x32 0.019 / 0.020, 128x128x64 0.030 / 0.026,
 // 256x256x128 0.079 / 0.068, 300x300x160 0.159 / 0.112, 270x360x180 0.194 /
-// 0.136, 384x384x256 0.332 / 0.247, 512x512x256 0.521 / 0.496, 1024x512x64
-// 0.240 / 0.243.  Calls against the three passes with built-in shapes:
-// Biggs-10 at 270x360x180 5.72 -> 4.04 ms, 8 chunks of up to 384x384x256 25.9 ->
-// 20.5 ms, OMW-2 at 512x512x256 2.42 -> 2.35 ms.
+// 0.136, 384x384x256 0.332 / 0.247, 512x512x256 0.520 / 0.507.  Calls against the
+// three passes with built-in shapes: Biggs-10 at 270x360x180 5.72 -> 4.02 ms, 8
+// chunks of up to 384x384x256 25.9 -> 20.7 ms, OMW-2 at 512x512x256 2.42 -> 2.31
+// ms.  HBM bytes there: column pass 0.86 GB, ratio 0.70, 1.07 and 1.03 times the
+// algorithmic ones.  Sizes whose three passes are faster keep them (default_fold,
+// pk_engine.hip).
 //
-// What bounds it: the column pass moves 3.4-4.2 TB/s; the ratio's row pass is
-// held by its arithmetic (about 100 vector instructions an element: two row
-// transforms, two splits, four dim-2 steps) where the tile leaves one block a CU
-// (512x512x256: 140 KB, 0.26 ms against 0.14 ms of bytes at the copy rate), so
-// nothing hides its load and store phases.
+// What bounds it: the column pass moves 3.4-4.2 TB/s.  Where the tiles leave one
+// block a CU (512x512x256: 140 and 147 KB) nothing hides a block's load and store
+// phases: the ratio's row pass takes 0.26 ms for 0.14 ms of vector instructions
+// (about 100 an element: two row transforms, two splits, four dim-2 steps) and
+// 0.15 ms of bytes at the copy rate, one after the other.
 #pragma once
 #include "pk_fft_dev.hpp"
 
@@ -140,8 +142,8 @@ __device__ __forceinline__ int fold_slot(const FoldX& f, int k) {
 // carries the rounding of its factors, and a power of one value m times that
 // value's: with stage_twiddle's powers of W^1 the error of OMW-2 against 64 bits
 // was up to 1.46 times the three passes' (64x64x32, 3.5e-7 against 2.4e-7).  Here
-// no power takes more than W^1 or W^2 and one of the table's W^4, W^8, W^12, and
-// R <= 4 and R = 8 read all from the table: 0.56-1.07 times the three passes'
+// a power is a table value, or W^1 or W^2 and one of the table's W^4, W^8, W^12 (the
+// last one of R = 12 and 16 takes three factors); R <= 4 and R = 8 read all from the table: 0.56-1.07 times the three passes'
 // error over 20 sizes, for up to 1.4 % of the time (8 chunks of up to 384x384x256,
 // Biggs-10, 20.4 -> 20.7 ms).  All radices from the table: no closer, 2-4 % slower.
 template <int R, bool INV>
